@@ -221,6 +221,18 @@ int pnfam_gpu_calc_hamiltonian_noalloc(pnfam_gpu_ctx *h, const double *d_in, dou
  *   unit_replicas  1..256: the per-unit entry points run their frequency in
  *                  that many batch slots (identical inputs) and return the last,
  *                  so that they take the launch paths of batches that size;
+ *                  once it is given (1 too), the FP64 grid stage of the
+ *                  per-unit calls runs the general kernels, whose launch-shape
+ *                  options (proj_*, fp64_density) it serves to compare;
+ *   fp64_grid      0 (default): on a basis whose wavefunction tables are
+ *                  products of a radial and an axial function (found from the
+ *                  tables when the context is created; the harmonic-oscillator
+ *                  bases all are) the FP64 grid stage contracts one direction
+ *                  at a time, in all solves and per-unit calls but
+ *                  calc_hamiltonian_noalloc; 1: always the general kernels,
+ *                  which contract over all grid points (results differ in
+ *                  summation order; read back fp64_separable: 1 where the
+ *                  first form is in use);
  *   mix_tau        one-product threshold of the mixed path (PNFAM_GPU_MIX_TAU);
  *   mix_hist64     1: the mixed path keeps its Broyden history in FP64;
  *   mix_drop       0: keep the Broyden pair formed across a refinement;

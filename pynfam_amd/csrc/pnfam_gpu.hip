@@ -1733,6 +1733,7 @@ __global__ void k_proj_sum(const double *__restrict__ part, int nsplit, int na, 
 }
 
 #include "factored.hpp"
+#include "separable.hpp"
 
 struct GreenArgs {
   const double *hqp;     // [w][4][nxy]
@@ -2360,6 +2361,7 @@ struct pnfam_gpu_ctx {
   // per-unit entry points: batch slots their one frequency runs in (option
   // unit_replicas), so that they take the batched launch paths
   int unit_reps = 1;
+  bool unit_general = false;   // unit_replicas given: the grid stage of the FP64 unit calls runs the general kernels
   std::vector<int> unit_act;
   // mixed-path options (environment defaults, pnfam_gpu_set_option)
   double mix_tau = 3e-3;        // one-product threshold (PNFAM_GPU_MIX_TAU)
@@ -2371,6 +2373,25 @@ struct pnfam_gpu_ctx {
   // per-unit Broyden hook (pnfam_gpu_broyden_step): history size and mixing in use
   int hook_M = -2;
   double hook_alpha = 0.0;
+  // FP64 grid stage on product grids (separable.hpp): the basis part, found when
+  // the context is created, and the plan of the operator's block structures
+  struct SepGroup { int cls, first, count; };   // radial function, members of the state list
+  bool sep_basis = false, sep_plan = false, sep_nomem = false;
+  int sep_nz = 0, sep_nr = 0, sep_ncls = 0;
+  std::vector<SepGroup> sep_groups;              // per (block, spin), in order of sep_gfirst
+  std::vector<int> sep_gfirst;                   // [2 nb + 1]
+  std::vector<int> sep_members;                  // local state indices
+  DevPtr d_sep_f, d_sep_fz;
+  DevPtr d_sep_keys, d_sep_tabs, d_sep_djobs, d_sep_pjobs;
+  DevPtr d_sep_slots[2], d_sep_elems[2];         // density, projection
+  int sep_nslot[2] = {0, 0}, sep_ndjob = 0, sep_npjob[2] = {0, 0}, sep_pjob0[2] = {0, 0};
+  int sep_ct[2] = {1, 1}, sep_ncg[2] = {1, 1};   // density, projection: column tiles per wave, column groups
+  SepAcc sep_acc{};
+  long sep_zstride = 0, sep_ystride = 0, sep_arows = 0;
+  double sep_flops_d = 0, sep_flops_p = 0;       // FLOP per point of the two halves; gen_: of the general kernels
+  double gen_flops_d = 0, gen_flops_p = 0;
+  DevPtr d_sep_zy, d_sep_part;                   // Z / Y and partial densities of a chunk of points
+  int fp64_grid = 0;                             // 0: the separable stage where there is a plan, 1: never
   // cross-term operators in the qp basis, g20 / g02 [nx][nxy], and their
   // contractions with every point's amplitudes [w][nx][2]
   int nx = 0;
@@ -2837,6 +2858,8 @@ int stage_hamiltonian_on(pnfam_gpu_ctx *h, int na, const int *act, const GridBuf
   // sector 0: rho_pn = m11 (slot 0), kappa+ = m12 (slot 1); sector 1: rho_np = m22 (3), kappa- = m21 (2)
   A.rho_slot[0] = 0; A.kap_slot[0] = 1; A.rho_slot[1] = gb.rho1; A.kap_slot[1] = gb.kap1;
   A.dens = gb.dens; A.act = act; A.skip = h->skip_slot;
+  h->flops_unit[K_DENSITY] = h->gen_flops_d;
+  h->flops_unit[K_PROJECT] = h->gen_flops_p;
   { Prof pr(h, K_DENSITY, na);
     if (h->basic_kernels) {
       note(h, "k_density");
@@ -2936,9 +2959,393 @@ int stage_hamiltonian_on(pnfam_gpu_ctx *h, int na, const int *act, const GridBuf
   return 0;
 }
 
+// ---- FP64 grid stage on product grids (separable.hpp) ------------------------
+constexpr int sep_pad8(int n) { return (n + 7) & ~7; }
+
+// Points along z of the product grid: the divisor of nghl for which the values
+// of a few states are rank-one matrices; 0 if there is none.
+int sep_axial_points(const pnfam_gpu_basis *b) {
+  const int G = b->nghl;
+  for (int nz = 2; nz <= G / 2; ++nz) {
+    if (G % nz || nz > SEP_MAX1D || G / nz > SEP_MAX1D) continue;
+    bool ok = true;
+    for (int k = 0; k < 3 && ok; ++k) {
+      const double *M = b->wf + (size_t)((long)k * (b->dqp - 1) / 2) * G;
+      int p = 0;
+      for (int i = 1; i < G; ++i)
+        if (std::fabs(M[i]) > std::fabs(M[p])) p = i;
+      const int rp = p / nz, zp = p % nz;
+      const double m = M[p], tol = 1e-12 * m * m;
+      ok = m != 0.0;
+      for (int i = 0; i < G && ok; ++i)
+        ok = std::fabs(M[i] * m - M[rp * nz + i % nz] * M[(i / nz) * nz + zp]) <= tol;
+    }
+    if (ok) return nz;
+  }
+  return 0;
+}
+
+// Factors of the wavefunction tables and the radial functions they share.
+// Leaves sep_basis false where the tables are no products.
+int sep_prepare(pnfam_gpu_ctx *h, const pnfam_gpu_basis *b) {
+  const int nz = sep_axial_points(b);
+  if (!nz) return 0;
+  const int nr = b->nghl / nz, D = b->dqp;
+  DevPtr dfr, dres;
+  int e;
+  if ((e = dfr.alloc((size_t)D * 4 * nr * 8)) || (e = dres.alloc((size_t)D * 8)) ||
+      (e = h->d_sep_fz.alloc((size_t)3 * D * sep_pad8(nz) * 8)))
+    return e;
+  SepFit S{};
+  S.tab[0] = h->d_wf.as<double>(); S.tab[1] = h->d_wfdr.as<double>(); S.tab[2] = h->d_wfdp.as<double>();
+  S.tab[3] = h->d_wfdz.as<double>(); S.tab[4] = h->d_wfd2.as<double>();
+  S.nz = nz; S.nr = nr; S.dqp = D; S.nzp = sep_pad8(nz); S.fr = dfr.as<double>(); S.fz = h->d_sep_fz.as<double>();
+  S.resid = dres.as<double>();
+  hipLaunchKernelGGL(k_sep_fit, dim3(D), dim3(256), 0, h->stream, S);
+  HIP_TRY(hipGetLastError());
+  std::vector<double> fr((size_t)D * 4 * nr), res(D);
+  HIP_TRY(hipMemcpyAsync(fr.data(), dfr.p, fr.size() * 8, hipMemcpyDeviceToHost, h->stream));
+  HIP_TRY(hipMemcpyAsync(res.data(), dres.p, res.size() * 8, hipMemcpyDeviceToHost, h->stream));
+  HIP_TRY(hipStreamSynchronize(h->stream));
+  for (double r : res)
+    if (!(r <= SEP_TOL)) return 0;
+  // radial functions equal to rounding (all four tables) form one class,
+  // represented by the mean of its members
+  std::vector<int> cls(D), first;
+  std::vector<int> cnt;
+  auto same = [&](int a, int c) {
+    for (int x = 0; x < 4; ++x) {
+      const double *u = &fr[((size_t)a * 4 + x) * nr], *v = &fr[((size_t)c * 4 + x) * nr];
+      double m = 0.0;
+      for (int r = 0; r < nr; ++r) m = std::max(m, std::fabs(v[r]));
+      for (int r = 0; r < nr; ++r)
+        if (!(std::fabs(u[r] - v[r]) <= SEP_TOL * m)) return false;
+    }
+    return true;
+  };
+  for (int a = 0; a < D; ++a) {
+    int c = -1;
+    for (size_t k = 0; k < first.size() && c < 0; ++k)
+      if (same(a, first[k])) c = (int)k;
+    if (c < 0) { c = (int)first.size(); first.push_back(a); cnt.push_back(0); }
+    cls[a] = c;
+    ++cnt[c];
+  }
+  const int nc = (int)first.size();
+  std::vector<double> f((size_t)4 * nc * nr, 0.0);
+  for (int a = 0; a < D; ++a)
+    for (int x = 0; x < 4; ++x)
+      for (int r = 0; r < nr; ++r) f[((size_t)x * nc + cls[a]) * nr + r] += fr[((size_t)a * 4 + x) * nr + r];
+  for (int x = 0; x < 4; ++x)
+    for (int c = 0; c < nc; ++c)
+      for (int r = 0; r < nr; ++r) f[((size_t)x * nc + c) * nr + r] /= cnt[c];
+  h->sep_groups.clear(); h->sep_members.clear();
+  h->sep_gfirst.assign(2 * h->nb + 1, 0);
+  for (int i = 0; i < h->nb; ++i)
+    for (int s = 0; s < 2; ++s) {
+      const int lo = s ? h->nsu[i] : 0, hi = s ? h->db[i] : h->nsu[i];
+      std::vector<int> order;
+      for (int k = lo; k < hi; ++k) order.push_back(k);
+      std::stable_sort(order.begin(), order.end(),
+                       [&](int a, int c) { return cls[h->isstart[i] + a] < cls[h->isstart[i] + c]; });
+      h->sep_gfirst[2 * i + s] = (int)h->sep_groups.size();
+      for (int k : order) {
+        const int c = cls[h->isstart[i] + k];
+        if ((int)h->sep_groups.size() == h->sep_gfirst[2 * i + s] || h->sep_groups.back().cls != c)
+          h->sep_groups.push_back({c, (int)h->sep_members.size(), 0});
+        h->sep_members.push_back(k);
+        ++h->sep_groups.back().count;
+      }
+    }
+  h->sep_gfirst[2 * h->nb] = (int)h->sep_groups.size();
+  if ((e = upload(h->d_sep_f, f.data(), f.size() * 8, h->stream))) return e;
+  HIP_TRY(hipStreamSynchronize(h->stream));   // pageable sources
+  h->sep_nz = nz; h->sep_nr = nr; h->sep_ncls = nc;
+  h->sep_basis = true;
+  return 0;
+}
+
+// Plan for the block structures of the operator: slots, tables of radial
+// products and the jobs of the four kernels.
+int sep_build(pnfam_gpu_ctx *h) {
+  h->sep_plan = false;
+  if (!h->sep_basis) return 0;
+  const int nz = h->sep_nz, nr = h->sep_nr, W = 2 * nz, nr4 = (nr + 3) & ~3;
+  const BlockMap *dm[4] = {&h->rspmap[0], &h->rspmap[1], &h->rspmap[3], &h->rspmap[2]};   // rho0, kap0, rho1, kap1
+  const BlockMap *pm[4] = {&h->hspmap[0], &h->hspmap[1], &h->hspmap[3], &h->hspmap[2]};   // h0, D0, h1, D1
+  const int out_slot[4] = {0, 1, 3, 2};
+  typedef std::vector<std::pair<int, int>> Keys;
+  struct Tab { int kind, sa, sb; Keys keys; bool d = false, p = false; size_t key0 = 0, rd = 0, rp = 0; };
+  std::vector<Tab> tabs;
+  auto groups = [&](int blk, int s) {
+    return std::make_pair(h->sep_gfirst[2 * blk + s], h->sep_gfirst[2 * blk + s + 1]);
+  };
+  // slots of one structure and pair of spins, in the order of (row, column) function
+  auto keys_of = [&](const BlockMap &m, int sa, int sb) {
+    Keys k;
+    for (auto &p : pair_list(m)) {
+      const auto ga = groups(p.x, sa), gb = groups(p.y, sb);
+      for (int i = ga.first; i < ga.second; ++i)
+        for (int j = gb.first; j < gb.second; ++j) k.push_back({h->sep_groups[i].cls, h->sep_groups[j].cls});
+    }
+    std::sort(k.begin(), k.end());
+    k.erase(std::unique(k.begin(), k.end()), k.end());
+    return k;
+  };
+  int dtab[16], ptab[16];
+  for (int q = 0; q < 16; ++q) {
+    const int mat = q >> 2, sa = (q >> 1) & 1, sb = q & 1, kind = mat & 1;
+    for (int side = 0; side < 2; ++side) {
+      Keys k = keys_of(side ? *pm[mat] : *dm[mat], sa, sb);
+      int t = -1;
+      for (size_t i = 0; i < tabs.size() && t < 0; ++i)
+        if (tabs[i].kind == kind && tabs[i].sa == sa && tabs[i].sb == sb && tabs[i].keys == k) t = (int)i;
+      if (t < 0) {
+        t = (int)tabs.size();
+        tabs.push_back({kind, sa, sb, std::move(k)});
+      }
+      (side ? tabs[t].p : tabs[t].d) = true;
+      (side ? ptab : dtab)[q] = t;
+    }
+  }
+  auto slot_id = [&](const Tab &t, int ca, int cb) {
+    return (int)(std::lower_bound(t.keys.begin(), t.keys.end(), std::make_pair(ca, cb)) - t.keys.begin());
+  };
+  std::vector<int2> keys;
+  size_t doubles = 0;
+  for (auto &t : tabs) {
+    const size_t n = t.keys.size();
+    const bool same = t.sa == t.sb;
+    t.key0 = keys.size();
+    for (auto &k : t.keys) keys.push_back(make_int2(k.first, k.second));
+    if (t.d) { t.rd = doubles; doubles += ((n + 3) & ~size_t(3)) * sep_row0(t.kind, same, SEP_NT, nr); }
+    if (t.p) { t.rp = doubles; doubles += ((n + 15) & ~size_t(15)) * sep_k0(t.kind, same, SEP_PT, nr4); }
+  }
+  int e;
+  if ((e = upload(h->d_sep_keys, keys.data(), std::max<size_t>(1, keys.size()) * sizeof(int2), h->stream)) ||
+      (e = h->d_sep_tabs.alloc(std::max<size_t>(1, doubles) * 8)))
+    return e;
+  double *tb = h->d_sep_tabs.as<double>();
+  for (auto &t : tabs) {
+    if (t.keys.empty()) continue;
+    const SepTab T{h->d_sep_keys.as<int2>() + t.key0, (int)t.keys.size(), t.kind, t.sa, t.sb, t.d ? tb + t.rd : nullptr,
+                   t.p ? tb + t.rp : nullptr};
+    hipLaunchKernelGGL(k_sep_rtab, dim3(512), dim3(256), 0, h->stream, T, h->d_sep_f.as<double>(), nr, h->sep_ncls);
+  }
+  HIP_TRY(hipGetLastError());
+  // column tiles per wave: at most five (20 accumulator tiles)
+  const int W8 = 2 * sep_pad8(nz);
+  for (int k = 0; k < 2; ++k) {
+    const int nct = ((k ? W8 : W) + 15) / 16;
+    h->sep_ncg[k] = (nct + 4) / 5;
+    h->sep_ct[k] = (nct + h->sep_ncg[k] - 1) / h->sep_ncg[k];
+  }
+  std::vector<SepSlot> slots[2];
+  std::vector<int4> elems[2];
+  std::vector<SepDJob> djobs;
+  std::vector<SepPJob> pjobs[2];
+  long zoff = 0, yoff = 0, arow = 0;
+  h->sep_flops_d = h->sep_flops_p = 0;
+  // the slots of one class with their elements; each slot takes `ld` doubles from `at` on
+  auto put_slots = [&](int side, int q, const Tab &T, const BlockMap &m, long at, long ld) {
+    const int mat = q >> 2, sa = (q >> 1) & 1, sb = q & 1;
+    std::vector<std::vector<int4>> el(T.keys.size());
+    for (auto &p : pair_list(m)) {
+      const auto ga = groups(p.x, sa), gb = groups(p.y, sb);
+      for (int i = ga.first; i < ga.second; ++i)
+        for (int j = gb.first; j < gb.second; ++j) {
+          const auto &A = h->sep_groups[i], &B = h->sep_groups[j];
+          auto &v = el[slot_id(T, A.cls, B.cls)];
+          for (int b = 0; b < B.count; ++b)
+            for (int a = 0; a < A.count; ++a) {
+              const int al = h->sep_members[A.first + a], bl = h->sep_members[B.first + b];
+              v.push_back(make_int4(p.z + al + bl * h->db[p.x], h->isstart[p.x] + al, h->isstart[p.y] + bl, 0));
+            }
+        }
+    }
+    for (size_t s = 0; s < el.size(); ++s) {
+      slots[side].push_back({(int)elems[side].size(), (int)el[s].size(), mat, (int)(at + (long)s * ld)});
+      elems[side].insert(elems[side].end(), el[s].begin(), el[s].end());
+    }
+  };
+  for (int q = 0; q < 16; ++q) {
+    const int mat = q >> 2, sa = (q >> 1) & 1, sb = q & 1, kind = mat & 1;
+    const bool same = sa == sb;
+    {   // densities
+      const Tab &T = tabs[dtab[q]];
+      const int n = (int)T.keys.size(), nt = kind ? 1 : SEP_NT, ld = sep_row0(kind, same, SEP_NT, nr);
+      put_slots(0, q, T, *dm[mat], zoff, (long)nt * W);
+      h->sep_acc.row[q] = n ? (int)arow : -1;
+      for (int t = 0; t < nt && n; ++t) {
+        const int r0 = sep_row0(kind, same, t, nr), r1 = sep_row0(kind, same, t + 1, nr);
+        for (int r = r0; r < r1; r += 64)
+          djobs.push_back({tb + T.rd, n, ld, r, std::min(4, (r1 - r) / 16), (int)(zoff + (long)t * W), nt * W,
+                           (int)arow + r, 0});
+        h->sep_flops_d += 2.0 * n * sep_rows(kind, same, t) * nr * W;
+      }
+      zoff += (long)n * nt * W;
+      arow += n ? ld : 0;
+    }
+    {   // projection
+      const Tab &T = tabs[ptab[q]];
+      const int n = (int)T.keys.size(), nt = kind ? 1 : SEP_PT, ld = (n + 15) & ~15;
+      put_slots(1, q, T, *pm[mat], yoff, (long)nt * W8);
+      for (int t = 0; t < nt && n; ++t) {
+        h->sep_flops_p += 2.0 * n * sep_terms(kind, same, t) * nr * W;
+        for (int v = 0; v < 2; ++v) {
+          const int rt = v ? 4 : 1;
+          for (int s = 0; s < ld; s += 16 * rt)
+            pjobs[v].push_back({tb + T.rp + (size_t)sep_k0(kind, same, t, nr4) * ld, ld, n, s,
+                                std::min(rt, (ld - s) / 16), sep_terms(kind, same, t), t, kind, sa, sb, mat >> 1,
+                                (int)(yoff + (long)t * W8), nt * W8});
+        }
+      }
+      yoff += (long)n * nt * W8;
+    }
+    // per element: the axial products of the densities and of the expansion
+    h->sep_flops_d += (kind ? 4.0 : 16.0) * nz * (double)dm[mat]->nelem(h->db) / 4;
+    h->sep_flops_p += (kind ? 4.0 : 20.0) * nz * (double)pm[mat]->nelem(h->db) / 4;
+    if (zoff > (1L << 30) || yoff > (1L << 30)) return 0;   // offsets are 32-bit: such a basis keeps the other kernels
+  }
+  // longest first, so that the last workgroups of a launch are short ones
+  std::stable_sort(djobs.begin(), djobs.end(), [](const SepDJob &a, const SepDJob &b) { return a.n * a.nrt > b.n * b.nrt; });
+  for (auto &v : pjobs)
+    std::stable_sort(v.begin(), v.end(), [](const SepPJob &a, const SepPJob &b) { return a.nc * a.nst > b.nc * b.nst; });
+  for (auto &v : slots)
+    std::stable_sort(v.begin(), v.end(), [](const SepSlot &a, const SepSlot &b) {
+      return (a.mat & 1) != (b.mat & 1) ? (a.mat & 1) < (b.mat & 1) : a.count > b.count;
+    });
+  std::vector<SepPJob> pj(pjobs[0]);
+  pj.insert(pj.end(), pjobs[1].begin(), pjobs[1].end());
+  for (int k = 0; k < 2; ++k) {
+    h->sep_nslot[k] = (int)slots[k].size();
+    if ((e = upload(h->d_sep_slots[k], slots[k].data(), std::max<size_t>(1, slots[k].size()) * sizeof(SepSlot), h->stream)) ||
+        (e = upload(h->d_sep_elems[k], elems[k].data(), std::max<size_t>(1, elems[k].size()) * sizeof(int4), h->stream)))
+      return e;
+  }
+  if ((e = upload(h->d_sep_djobs, djobs.data(), std::max<size_t>(1, djobs.size()) * sizeof(SepDJob), h->stream)) ||
+      (e = upload(h->d_sep_pjobs, pj.data(), std::max<size_t>(1, pj.size()) * sizeof(SepPJob), h->stream)))
+    return e;
+  HIP_TRY(hipStreamSynchronize(h->stream));   // pageable sources
+  h->sep_ndjob = (int)djobs.size();
+  for (int v = 0; v < 2; ++v) {
+    h->sep_pjob0[v] = v ? (int)pjobs[0].size() : 0;
+    h->sep_npjob[v] = (int)pjobs[v].size();
+  }
+  h->sep_zstride = zoff; h->sep_ystride = yoff; h->sep_arows = arow;
+  h->sep_plan = !djobs.empty() && !pj.empty();
+  return 0;
+}
+
+bool sep_active(const pnfam_gpu_ctx *h) {
+  return h->sep_plan && h->fp64_grid == 0 && !h->basic_kernels && !h->sep_nomem;
+}
+
+// Points a pass of the separable stage takes at once, and the splits of its
+// density contraction: with few points the slots are split so that about 2 048
+// waves run.
+constexpr size_t SEP_CHUNK_BYTES = size_t(1) << 30;
+int sep_chunk(const pnfam_gpu_ctx *h, int na) {
+  const size_t per = (size_t)std::max(h->sep_zstride, h->sep_ystride) * 8;
+  return (int)std::max<size_t>(1, std::min<size_t>((size_t)na, SEP_CHUNK_BYTES / std::max<size_t>(1, per)));
+}
+int sep_split(const pnfam_gpu_ctx *h, int nc, bool split) {
+  if (!split) return 1;
+  const long waves = (long)h->sep_ndjob * h->sep_ncg[0] * nc;
+  return (int)std::max<long>(1, std::min<long>(16, 2048 / std::max<long>(1, waves)));
+}
+
+// Device memory of a pass over na points, before any launch (a captured pass
+// cannot allocate).
+int sep_workspace(pnfam_gpu_ctx *h, int na) {
+  const int nc = sep_chunk(h, na);
+  if (int e = h->d_sep_zy.alloc((size_t)nc * std::max(h->sep_zstride, h->sep_ystride) * 8)) return e;
+  // split counts fall as the points rise: the most partial sums any count up to nc needs
+  long parts = 0;
+  for (int n = 1; n <= nc; ++n) parts = std::max(parts, (long)n * sep_split(h, n, true));
+  return h->d_sep_part.alloc((size_t)parts * h->sep_arows * 2 * h->sep_nz * 8);
+}
+
+// Densities, fields and projection through the separable kernels.
+int stage_hamiltonian_sep(pnfam_gpu_ctx *h, int na, const int *act, const GridBufs &gb) {
+  SepArgs A{};
+  A.nz = h->sep_nz; A.nr = h->sep_nr; A.dqp = h->dqp; A.nxy = h->nxy;
+  A.nzp = sep_pad8(A.nz); A.fz = h->d_sep_fz.as<double>();
+  A.rsp = gb.rsp; A.dens = gb.dens; A.flds = gb.flds; A.hsp = gb.hsp; A.wdcori = h->d_wdcori.as<double>();
+  A.slot_of[0] = 0; A.slot_of[1] = 1; A.slot_of[2] = gb.rho1; A.slot_of[3] = gb.kap1;
+  A.zy = h->d_sep_zy.as<double>(); A.zstride = h->sep_zstride; A.ystride = h->sep_ystride;
+  A.acc = h->d_sep_part.as<double>(); A.astride = h->sep_arows * 2 * h->sep_nz; A.skip = h->skip_slot;
+  h->flops_unit[K_DENSITY] = h->sep_flops_d;
+  h->flops_unit[K_PROJECT] = h->sep_flops_p;
+  const int C = sep_chunk(h, na), G = h->nghl;
+  for (int c0 = 0; c0 < na; c0 += C) {
+    const int nc = std::min(C, na - c0);
+    A.act = act + c0;
+    A.na = nc;
+    { Prof pr(h, K_DENSITY, nc);
+      const int ns = sep_split(h, nc, gb.split);
+      note(h, "k_sep_dens", h->sep_ct[0], ns);
+      const int zt = (h->sep_nz + 15) / 16, zg = (zt + 2) / 3;
+      const dim3 zgrid((h->sep_nslot[0] + 3) / 4, (nc + 7) / 8, zg);
+      const SepSlot *sl = h->d_sep_slots[0].as<SepSlot>();
+      const int4 *el = h->d_sep_elems[0].as<int4>();
+      switch ((zt + zg - 1) / zg) {
+        case 1: hipLaunchKernelGGL(k_sep_z<1>, zgrid, dim3(256), 0, h->stream, A, sl, el, h->sep_nslot[0]); break;
+        case 2: hipLaunchKernelGGL(k_sep_z<2>, zgrid, dim3(256), 0, h->stream, A, sl, el, h->sep_nslot[0]); break;
+        default: hipLaunchKernelGGL(k_sep_z<3>, zgrid, dim3(256), 0, h->stream, A, sl, el, h->sep_nslot[0]); break;
+      }
+      const dim3 grid(h->sep_ndjob, nc, h->sep_ncg[0] * ns);
+#define SEP_D(CT) hipLaunchKernelGGL(k_sep_dens<CT>, grid, dim3(64), 0, h->stream, A, h->d_sep_djobs.as<SepDJob>(), h->sep_ncg[0], ns)
+      switch (h->sep_ct[0]) {
+        case 1: SEP_D(1); break;
+        case 2: SEP_D(2); break;
+        case 3: SEP_D(3); break;
+        case 4: SEP_D(4); break;
+        default: SEP_D(5); break;
+      }
+#undef SEP_D
+      if (ns > 1)
+        hipLaunchKernelGGL(k_sep_sum, grid1((size_t)nc * A.astride, 256), dim3(256), 0, h->stream, A.acc, ns,
+                           (long)nc * A.astride);
+      hipLaunchKernelGGL(k_sep_combine, dim3((G + 127) / 128, nc, 2), dim3(128), 0, h->stream, A, h->sep_acc);
+    }
+    if (int e = stage_fields(h, nc, A.act, gb.dens, gb.flds)) return e;
+    if (!(h->zero_skip && h->proj_cover)) {
+      Prof pr(h, K_ZERO, nc);
+      hipLaunchKernelGGL(k_zero_slots, dim3(64, nc), dim3(256), 0, h->stream, gb.hsp, A.act, 8, 0, 8, h->nxy,
+                         h->skip_slot);
+    }
+    { Prof pr(h, K_PROJECT, nc);
+      const int v = nc >= 8 ? 1 : 0;   // four slot tiles per wave from eight points, one below
+      note(h, "k_sep_proj", h->sep_ct[1], v ? 4 : 1);
+      const dim3 grid(h->sep_npjob[v], nc, h->sep_ncg[1]);
+      const SepPJob *pj = h->d_sep_pjobs.as<SepPJob>() + h->sep_pjob0[v];
+#define SEP_P(CT)                                                                                    \
+  do {                                                                                               \
+    if (v) hipLaunchKernelGGL((k_sep_proj<CT, 4>), grid, dim3(64), 0, h->stream, A, pj);             \
+    else hipLaunchKernelGGL((k_sep_proj<CT, 1>), grid, dim3(64), 0, h->stream, A, pj);               \
+  } while (0)
+      switch (h->sep_ct[1]) {
+        case 1: SEP_P(1); break;
+        case 2: SEP_P(2); break;
+        case 3: SEP_P(3); break;
+        case 4: SEP_P(4); break;
+        default: SEP_P(5); break;
+      }
+#undef SEP_P
+      hipLaunchKernelGGL(k_sep_expand, dim3((h->sep_nslot[1] + 3) / 4, (nc + 7) / 8), dim3(256), 0, h->stream, A,
+                         h->d_sep_slots[1].as<SepSlot>(), h->d_sep_elems[1].as<int4>(), h->sep_nslot[1]);
+    }
+  }
+  HIP_TRY(hipGetLastError());
+  return 0;
+}
+
 int stage_hamiltonian(pnfam_gpu_ctx *h, int na, const int *act) {
   const GridBufs gb{h->d_rsp.as<double>(), 3, 2, h->d_dens.as<double>(), h->d_flds.as<double>(), h->d_hsp.as<double>(),
                     h->few_split_on != 0};
+  // without memory for the separable stage's intermediates the general kernels run
+  if (sep_active(h) && sep_workspace(h, na) == 0) return stage_hamiltonian_sep(h, na, act, gb);
   return stage_hamiltonian_on(h, na, act, gb);
 }
 
@@ -3757,6 +4164,7 @@ int pnfam_gpu_create(const pnfam_gpu_basis *b, pnfam_gpu_ctx **out) {
       (e = upload(h->d_ns, h->ns.data(), (size_t)b->dqp * 4, h->stream)))
     return e;
   HIP_TRY(hipStreamSynchronize(h->stream));
+  if ((e = sep_prepare(h.get(), b))) return e;
   *out = h.release();
   return 0;
 }
@@ -3987,10 +4395,13 @@ int pnfam_gpu_set_operator(pnfam_gpu_ctx *h, int32_t beta_minus, const int32_t *
     const double nr1 = (double)h->rspmap[3].nelem(db), nk1 = (double)h->rspmap[2].nelem(db);
     h->flops_unit[K_TRIPROD_Q2S] = q2s;
     h->flops_unit[K_TRIPROD_S2Q] = s2q;
-    h->flops_unit[K_DENSITY] = G * (16.0 * (nr0 + nr1) + 4.0 * (nk0 + nk1));
-    h->flops_unit[K_PROJECT] = G * (20.0 * (double)(h->hspmap[0].nelem(db) + h->hspmap[3].nelem(db)) +
-                                    4.0 * (double)(h->hspmap[1].nelem(db) + h->hspmap[2].nelem(db)));
+    h->gen_flops_d = G * (16.0 * (nr0 + nr1) + 4.0 * (nk0 + nk1));
+    h->gen_flops_p = G * (20.0 * (double)(h->hspmap[0].nelem(db) + h->hspmap[3].nelem(db)) +
+                          4.0 * (double)(h->hspmap[1].nelem(db) + h->hspmap[2].nelem(db)));
+    h->flops_unit[K_DENSITY] = h->gen_flops_d;
+    h->flops_unit[K_PROJECT] = h->gen_flops_p;
   }
+  if ((e = sep_build(h))) return e;
   h->have_op = true;
   h->cap = 0;
   h->hist_cap = -1;
@@ -4095,7 +4506,11 @@ static int upload_args(pnfam_gpu_ctx *h, DevPtr &dst, const double *in) {
 
 static int unit_hamiltonian(pnfam_gpu_ctx *h) {
   const int R = h->unit_reps;
-  if (h->unit_precision == PNFAM_GPU_FP64) return stage_hamiltonian(h, R, h->d_act.as<int>());
+  if (h->unit_precision == PNFAM_GPU_FP64) {
+    const GridBufs gb{h->d_rsp.as<double>(), 3, 2, h->d_dens.as<double>(), h->d_flds.as<double>(),
+                      h->d_hsp.as<double>(), h->few_split_on != 0};
+    return h->unit_general ? stage_hamiltonian_on(h, R, h->d_act.as<int>(), gb) : stage_hamiltonian(h, R, h->d_act.as<int>());
+  }
   if (int e = mix_prepare(h)) return e;
   return stage_hamiltonian_lowp(h, R, h->d_act.as<int>(), R);
 }
@@ -4295,6 +4710,7 @@ static int solve_core(pnfam_gpu_ctx *h, int32_t npts, const double *re_w, const 
     if (int e = mix_prepare(h)) return e;
   const long nxy = h->nxy, N = 4 * nxy;
   h->bs.valid = false;
+  h->sep_nomem = false;
   h->hook_M = -2;   // the Broyden hook's history shares this workspace
   // graph replay of the FP64 iteration (option graph): one more slot, the
   // spare one the replays give the entries of retired points
@@ -4437,6 +4853,8 @@ static int solve_core(pnfam_gpu_ctx *h, int32_t npts, const double *re_w, const 
     int nslots = 0;
     for (int w = 0; w < npts; ++w) nslots += b.done[w] ? 0 : 1;
     if (nslots == 0) { iter = it0; return 0; }
+    // (without memory for the separable stage every capture takes the general kernels)
+    h->sep_nomem = sep_active(h) && sep_workspace(h, nslots) != 0;
     int *dact = h->d_act.as<int>();
     int *ctl = h->d_gctl.as<int>();
     auto body = [&](int ns) -> int {
@@ -4805,6 +5223,7 @@ int pnfam_gpu_set_option(pnfam_gpu_ctx *h, const char *name, double value) {
   if (n == "unit_replicas") {
     if (value < 1 || value > 256 || value != std::floor(value)) return fail(PNFAM_GPU_EINVAL, "unit_replicas in 1..256");
     h->unit_reps = (int)value;
+    h->unit_general = true;
   } else if (n == "mix_tau") {
     if (!(value >= 0)) return fail(PNFAM_GPU_EINVAL, "mix_tau must be >= 0");
     h->mix_tau = value;
@@ -4848,6 +5267,9 @@ int pnfam_gpu_set_option(pnfam_gpu_ctx *h, const char *name, double value) {
   } else if (n == "few_split") {
     if (value != 0 && value != 1) return fail(PNFAM_GPU_EINVAL, "few_split: 0 or 1");
     h->few_split_on = (int)value;
+  } else if (n == "fp64_grid") {
+    if (value != 0 && value != 1) return fail(PNFAM_GPU_EINVAL, "fp64_grid: 0 (separable where the basis allows) or 1 (general)");
+    h->fp64_grid = (int)value;
   } else if (n == "proj_stages") {
     if (value != 1 && value != 2) return fail(PNFAM_GPU_EINVAL, "proj_stages: 1 or 2");
     h->proj_ns = (int)value;
@@ -4896,6 +5318,8 @@ int pnfam_gpu_get_option(pnfam_gpu_ctx *h, const char *name, double *value) {
   else if (n == "proj_stages") *value = h->proj_ns;
   else if (n == "graph") *value = h->graph_mode;
   else if (n == "few_split") *value = h->few_split_on;
+  else if (n == "fp64_grid") *value = h->fp64_grid;
+  else if (n == "fp64_separable") *value = sep_active(h) ? 1 : 0;
   else if (n == "graph_launches") *value = (double)h->graph_launches;
   else if (n == "graph_captures") *value = (double)h->graph_captures;
   else if (n == "graph_capture_ms") *value = h->graph_capture_ms;
