@@ -150,95 +150,192 @@ __global__ void __launch_bounds__(256) k_triprod(const Group *__restrict__ group
   }
 }
 
-constexpr int TP_MAXCT = 8;    // column tiles of 16 per strip (block sizes up to 128)
-constexpr int TP_MERGE_N = 8;  // at most this many points: one triple-product launch over all tile classes
+// Keeps the loads of the next step above the products of the current one: nothing
+// in the program orders the two, and the compiler otherwise sinks each load to
+// its use in the next trip of the loop, where its latency is not hidden.
+__device__ inline void loads_first() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
 
-// Block triple products on the matrix cores.  One wave per (group, 16-row
-// strip of the output block, frequency): T_strip = s op(A)_strip op(B) is
-// accumulated over column tiles with v_mfma_f64_16x16x4, parked in LDS, and
-// multiplied by op(C); all terms of the group accumulate in registers.
-// Instantiated per number of 16-column tiles NCT (groups are sorted by it on
-// the host), so tile loops carry no branches and operand loads of a K step
-// issue together from clamped, always valid addresses.
-template <int NCT>
-__global__ void __launch_bounds__(64) k_triprod_mfma(const Group *__restrict__ groups, const Term *__restrict__ terms,
-                                                     const double *__restrict__ m0, const double *__restrict__ m1,
-                                                     const double *__restrict__ m2, const double *__restrict__ m3,
-                                                     const double *__restrict__ bbase, long bstride,
-                                                     double *__restrict__ obase, long ostride,
-                                                     const int *__restrict__ act, long nxy, int skip) {
-  constexpr int PITCH = 16 * NCT + 1;
-  __shared__ double sT[16 * PITCH];
+// Buffer of n doubles at a uniform p: loads with one address register (offsets of
+// the lanes; soff: a uniform offset on top), zero past the end.
+__device__ inline __amdgpu_buffer_rsrc_t rsrc64(const double *p, int n) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(p), 0, 8 * n, 0x00020000);
+}
+__device__ inline double load64(__amdgpu_buffer_rsrc_t r, int off, int soff) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, 8 * off, 8 * soff, 0));
+}
+
+constexpr int TP_MAXCT = 8;    // column tiles of 16 per strip (block sizes up to 128)
+constexpr int TP_MERGE_N = 8;  // at most this many points: one launch over all tile classes (bf16 triple products, projection)
+constexpr int TP_SPLIT_N = 4;  // at most this many points: FP64 triple products in one launch, a strip's columns on four waves
+
+// Resident matrices of the FP64 triple products: every block zero-padded to a
+// pitch P of 32 k, as stored (cm) and transposed (rm), so that op(A) is read with
+// its rows and op(C) with its columns along the lanes, aligned and unmasked.
+struct Tp64 {
+  const double *cm, *rm;
+  long mstride;          // doubles per matrix
+};
+
+__global__ void k_tp_pack(const double *__restrict__ m, const int4 *__restrict__ blocks, double *__restrict__ cm,
+                          double *__restrict__ rm) {
+  const int4 b = blocks[blockIdx.y];    // FP64 offset, padded offset, d, P
+  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < b.w * b.w; e += gridDim.x * blockDim.x) {
+    const int i = e % b.w, j = e / b.w;
+    const bool in = i < b.z && j < b.z;
+    cm[b.y + e] = in ? m[b.x + i + (size_t)j * b.z] : 0.0;
+    rm[b.y + e] = in ? m[b.x + j + (size_t)i * b.z] : 0.0;
+  }
+}
+
+// Block triple products on the matrix cores: the strips (16 rows) of an output
+// block on the waves of a workgroup, per group and frequency.
+//
+// A strip's first product is formed transposed, T^T(j, i) = sum_k op(B)(k, j)
+// op(A)(i, k): register v of tile c then holds T(i, 16 c + 4 v + lane / 16) for
+// i = lane % 16, which is the A operand of the second product's step
+// l = 16 c + 4 v, so T needs neither LDS nor a barrier.
+// op(B) and op(C), which all strips read, go through LDS in chunks of 16 rows,
+// the next chunk's loads in flight during the products of this one.  Read
+// straight into the operand layout, a matrix whose rows are contiguous gives
+// every lane a cache line of its own; the L1 then serves one lane a cycle, and
+// that, not the matrix rate, bound the kernel (counters: 0.7 to 0.9 L1 accesses
+// per cycle and CU, 27 to 29 per load, matrix cores busy 43 % of the time).
+// op(A), with its rows along the lanes, is read from the packed copies.  Buffer
+// loads keep an address in one register, which lets three waves of up to 96
+// columns (four of up to 64) share a SIMD.
+// N_sh = 16, both term sets of a stage at 128 points: 1.55 ms (0.87 ms at the
+// peak matrix rate), 2.4 ms with the operands read straight from memory and the
+// term sets in launches of their own.
+// NCT: 16-column tiles of the launch's groups; NW: waves.
+template <int NCT, int NW>
+__global__ void __launch_bounds__(64 * NW, NCT <= 4 ? 4 : (NCT <= 6 || (NCT == 7 && NW == 4) ? 3 : 2))
+    k_triprod_mfma(const Group *__restrict__ groups, const Term *__restrict__ terms, Tp64 M,
+                   const double *__restrict__ bbase, long bstride, double *__restrict__ obase, long ostride,
+                   const int *__restrict__ act, long nxy, int skip) {
+  constexpr int PJ = 16 * NCT + 1;   // chunk row pitch: odd, so that neither a column written nor four rows read collide much
+  __shared__ double buf[2][16 * PJ];
   const Group g = groups[blockIdx.x];
-  const int strip = blockIdx.z;
   const int w = act ? act[blockIdx.y] : (int)blockIdx.y;
   if (w == skip) return;
-  const int i0 = strip * 16;
-  if (i0 >= g.nrow) return;                       // uniform per wave
-  const int lane = threadIdx.x, mi = lane & 15, mk = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, mi = lane & 15, mk = lane >> 4;
+  constexpr int nth = 64 * NW;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i0 = 16 * ((int)blockIdx.z * NW + wv);
+  const bool on = i0 < g.nrow;               // waves past the block load and wait with the others
   const double *B = bbase + (size_t)w * bstride;
-  double *O = obase + (size_t)w * ostride + (size_t)g.out_slot * nxy + g.out_off;
+  // A chunk is 16 rows by 16 NCT columns, in runs of 16 values: thread group u0
+  // (16 threads) takes the runs u0 + 4 NW i.  All addresses are one register plus
+  // what is uniform or a constant.
+  constexpr int NG = 4 * NW, NL = 16 * NCT / NG;
+  const int l16 = tid & 15, u0 = tid >> 4;
   v4d acc[NCT];
 #pragma unroll
   for (int c = 0; c < NCT; ++c) acc[c] = v4d{0, 0, 0, 0};
-  const int irow = i0 + mi;                      // operand row of op(A) for this lane
-  const bool irow_ok = irow < g.nrow;
-  const int irc = irow_ok ? irow : 0;
   for (int t = 0; t < g.count; ++t) {
     const Term tm = terms[g.first + t];
-    const double *A = (tm.a_id == 0 ? m0 : tm.a_id == 1 ? m1 : tm.a_id == 2 ? m2 : m3) + tm.a_off;
-    const double *Bb = B + (size_t)tm.b_slot * nxy + tm.b_off;
-    const double *C = (tm.c_id == 0 ? m0 : tm.c_id == 1 ? m1 : tm.c_id == 2 ? m2 : m3) + tm.c_off;
-    const int nda = tm.nda, ndc = tm.ndc;
-    // column indices of this lane per tile, clamped into the block
-    int jc[NCT];
-    double jm[NCT];
+    const int nda = tm.nda, ndc = tm.ndc, Pa = (nda + 31) & ~31, Pc = (ndc + 31) & ~31;
+    const __amdgpu_buffer_rsrc_t Ap =
+        rsrc64((tm.ta ? M.rm : M.cm) + tm.a_id * M.mstride + tm.pad0 + (on ? i0 : 0), Pa * Pa - (on ? i0 : 0));
+    const __amdgpu_buffer_rsrc_t Cp = rsrc64((tm.tc ? M.cm : M.rm) + tm.c_id * M.mstride + tm.pad1, Pc * Pc);
+    // Rows and columns of op(B) past the block: zeros past its end (the buffer's
+    // bound), else other values of the same block; the padding of A and C takes
+    // both out.
+    const __amdgpu_buffer_rsrc_t Bb = rsrc64(B + (size_t)tm.b_slot * nxy + tm.b_off, nda * ndc);
+    // stored with its columns contiguous (tb): run u is row u % 16, columns 16 (u / 16)
+    // to + 15; else column u, 16 rows
+    const int ldb = tm.ldb, bk = tm.tb ? ldb : 1, bc = tm.tb ? 16 : 16 * ldb;
+    const int bd = tm.tb ? u0 * PJ + l16 : l16 * PJ + u0, br = tm.tb ? PJ : 1;
+    double st[NL];
+    auto bload = [&](int k0) {
 #pragma unroll
-    for (int c = 0; c < NCT; ++c) {
-      const int j = c * 16 + mi;
-      jc[c] = j < ndc ? j : 0;
-      jm[c] = j < ndc ? 1.0 : 0.0;
-    }
-    // phase 1: T_strip = s op(A)[i0:i0+16, :] op(B).  The 0/1 factors (not
-    // selects) keep every load unconditional; clamped addresses hold finite data.
+      for (int i = 0; i < NL; ++i)
+        st[i] = load64(Bb, u0 * ldb + l16 + k0 * bk + NG * i % 16 * ldb + NG * i / 16 * bc, 0);
+    };
+    auto bstore = [&](double *d) {
+#pragma unroll
+      for (int i = 0; i < NL; ++i) d[bd + NG * i % 16 * br + NG * i / 16 * 16] = st[i];
+    };
+    auto cload = [&](int l0) {
+#pragma unroll
+      for (int i = 0; i < NL; ++i) st[i] = load64(Cp, u0 * Pc + l16, (l0 + NG * i % 16) * Pc + NG * i / 16 * 16);
+    };
+    auto cstore = [&](double *d) {
+#pragma unroll
+      for (int i = 0; i < NL; ++i) d[u0 * PJ + l16 + NG * i % 16 * PJ + NG * i / 16 * 16] = st[i];
+    };
     v4d T[NCT];
 #pragma unroll
     for (int c = 0; c < NCT; ++c) T[c] = v4d{0, 0, 0, 0};
-    for (int k0 = 0; k0 < nda; k0 += 4) {
-      const int k = k0 + mk;
-      const bool kok = k < nda;
-      const int kc = kok ? k : 0;
-      const double km = kok ? 1.0 : 0.0;
-      const double av =
-          (tm.ta ? A[kc + (size_t)irc * nda] : A[irc + (size_t)kc * nda]) * (irow_ok ? km : 0.0);
-      double bv[NCT];
+    double an[4];
+    auto aload = [&](int k0) {
 #pragma unroll
-      for (int c = 0; c < NCT; ++c)
-        bv[c] = (tm.tb ? Bb[jc[c] + (size_t)kc * tm.ldb] : Bb[kc + (size_t)jc[c] * tm.ldb]) * (km * jm[c]);
-#pragma unroll
-      for (int c = 0; c < NCT; ++c) T[c] = mfma64(av, bv[c], T[c]);
-    }
-    // park s*T in LDS: D[i][j] lives in lane j + 16 (i % 4), register i / 4
-#pragma unroll
-    for (int c = 0; c < NCT; ++c)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) sT[(4 * v + mk) * PITCH + c * 16 + mi] = tm.s * T[c][v];
+      for (int s = 0; s < 4; ++s) an[s] = load64(Ap, mk * Pa + mi, (k0 + 4 * s) * Pa);
+    };
+    bload(0);
+    aload(0);
+    __syncthreads();                         // the previous term's last chunk has been read
+    bstore(buf[0]);
     __syncthreads();
-    // phase 2: acc += T_strip op(C)
-    for (int l0 = 0; l0 < ndc; l0 += 4) {
-      const int l = l0 + mk;
-      const bool lok = l < ndc;
-      const int lc = lok ? l : 0;
-      const double tv = sT[mi * PITCH + lc] * (lok ? 1.0 : 0.0);
-      double cv[NCT];
+    int cur = 0, k0 = 0;
+    for (; k0 + 16 < nda; k0 += 16) {
+      double a[4];
 #pragma unroll
-      for (int c = 0; c < NCT; ++c)
-        cv[c] = (tm.tc ? C[jc[c] + (size_t)lc * ndc] : C[lc + (size_t)jc[c] * ndc]) * jm[c];
+      for (int s = 0; s < 4; ++s) a[s] = an[s];
+      bload(k0 + 16);
+      aload(k0 + 16);
+      loads_first();
+      const double *d = buf[cur];
 #pragma unroll
-      for (int c = 0; c < NCT; ++c) acc[c] = mfma64(tv, cv[c], acc[c]);
+      for (int s = 0; s < 4; ++s) {
+#pragma unroll
+        for (int c = 0; c < NCT; ++c) T[c] = mfma64(d[(4 * s + mk) * PJ + 16 * c + mi], a[s], T[c]);
+        if (NCT > 3) __builtin_amdgcn_sched_barrier(0);
+      }
+      cur ^= 1;
+      bstore(buf[cur]);
+      __syncthreads();
     }
+    cload(0);
+    loads_first();
+    {
+      const double *d = buf[cur];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        if (s > 0 && k0 + 4 * s >= nda) break;
+#pragma unroll
+        for (int c = 0; c < NCT; ++c) T[c] = mfma64(d[(4 * s + mk) * PJ + 16 * c + mi], an[s], T[c]);
+        if (NCT > 3) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    cur ^= 1;
+    cstore(buf[cur]);
     __syncthreads();
+#pragma unroll
+    for (int c = 0; c < NCT; ++c) {
+      if (c + 1 < NCT) cload(16 * (c + 1));
+      loads_first();
+      const double *d = buf[cur];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        if (c == NCT - 1 && v > 0 && 16 * c + 4 * v >= ndc) break;   // only the last tile may end early
+        const double a = tm.s * T[c][v];
+#pragma unroll
+        for (int q = 0; q < NCT; ++q)
+          acc[q] = mfma64(a, d[(4 * v + mk) * PJ + 16 * q + mi], acc[q]);
+        if (NCT > 3) __builtin_amdgcn_sched_barrier(0);
+      }
+      cur ^= 1;
+      if (c + 1 < NCT) {
+        cstore(buf[cur]);
+        __syncthreads();
+      }
+    }
   }
+  if (!on) return;
+  double *O = obase + (size_t)w * ostride + (size_t)g.out_slot * nxy + g.out_off;
 #pragma unroll
   for (int c = 0; c < NCT; ++c) {
     const int j = c * 16 + mi;
@@ -246,6 +343,149 @@ __global__ void __launch_bounds__(64) k_triprod_mfma(const Group *__restrict__ g
     for (int v = 0; v < 4; ++v) {
       const int i = i0 + 4 * v + mk;
       if (i < g.nrow && j < g.ncol) O[i + (size_t)j * g.nrow] = acc[c][v];
+    }
+  }
+}
+
+// The same for the fewest points: one strip per workgroup, its column tiles dealt
+// to four waves (tile c to wave c % 4), of T for up to two terms, then of the
+// output, so that the chains run side by side and every sum keeps its order (and
+// its bits).  A wave turns its tiles of op(B) over in an LDS patch of its own;
+// T passes between the waves in the layout in which they read it.
+// N_sh = 16, one point: 50 us a stage, 141 us with the terms one after another
+// on one wave and re and im in launches of their own.
+template <int NCT>
+__global__ void __launch_bounds__(256, 3) k_triprod_split(const Group *__restrict__ groups,
+                                                          const Term *__restrict__ terms, Tp64 M,
+                                                          const double *__restrict__ bbase, long bstride,
+                                                          double *__restrict__ obase, long ostride,
+                                                          const int *__restrict__ act, long nxy, int skip) {
+  constexpr int NT = (NCT + 3) / 4, TS = 2;      // tiles per wave; terms per pass
+  __shared__ double tl[TS * 4 * NT * 256];
+  __shared__ double patch[4 * NT * 16 * 17];
+  const Group g = groups[blockIdx.x];
+  const int w = act ? act[blockIdx.y] : (int)blockIdx.y;
+  const int lane = threadIdx.x & 63, mi = lane & 15, mk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int i0 = 16 * (int)blockIdx.z;
+  if (w == skip || i0 >= g.nrow) return;          // uniform per workgroup
+  const double *B = bbase + (size_t)w * bstride;
+  double *d = patch + wave * NT * 16 * 17;
+  v4d acc[NT];
+#pragma unroll
+  for (int u = 0; u < NT; ++u) acc[u] = v4d{0, 0, 0, 0};
+  for (int t0 = 0; t0 < g.count; t0 += TS) {
+    const int nt = min(TS, g.count - t0);
+    const Term *tp = terms + g.first + t0;
+    // loads of the next 16 k, across the ends of the terms
+    Term tm = tp[0];
+    __amdgpu_buffer_rsrc_t Ap, Bb, Cp;
+    double an[4], bn[NT][4], cn[4][NT];
+    auto open_ab = [&](int t) {
+      tm = tp[t];
+      const int Pa = (tm.nda + 31) & ~31;
+      Ap = rsrc64((tm.ta ? M.rm : M.cm) + tm.a_id * M.mstride + tm.pad0 + i0, Pa * Pa - i0);
+      // past the block: zeros or other values of it, as in k_triprod_mfma
+      Bb = rsrc64(B + (size_t)tm.b_slot * nxy + tm.b_off, tm.nda * tm.ndc);
+    };
+    auto load_ab = [&](int k0) {
+      const int Pa = (tm.nda + 31) & ~31, bk = tm.tb ? tm.ldb : 1, bj = tm.tb ? 1 : tm.ldb;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) an[s] = load64(Ap, mk * Pa + mi, (k0 + 4 * s) * Pa);
+#pragma unroll
+      for (int u = 0; u < NT; ++u)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+          bn[u][s] = load64(Bb, mk * tm.ldb + mi + 4 * s * tm.ldb + k0 * bk + 16 * (wave + 4 * u) * bj, 0);
+    };
+    auto open_c = [&](int t) {
+      tm = tp[t];
+      const int Pc = (tm.ndc + 31) & ~31;
+      // columns past the block's padding read the next row: of output tiles that are not stored
+      Cp = rsrc64((tm.tc ? M.cm : M.rm) + tm.c_id * M.mstride + tm.pad1, Pc * Pc);
+    };
+    auto load_c = [&](int l0) {
+      const int Pc = (tm.ndc + 31) & ~31;
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) cn[v][u] = load64(Cp, mk * Pc + mi, (l0 + 4 * v) * Pc + 16 * (wave + 4 * u));
+    };
+    open_ab(0);
+    load_ab(0);
+    for (int t = 0; t < nt; ++t) {
+      const int nda = tm.nda, dw = tm.tb ? mk * 17 + mi : mi * 17 + mk, ds = tm.tb ? 4 * 17 : 4;
+      const double sc = tm.s;
+      v4d T[NT];
+#pragma unroll
+      for (int u = 0; u < NT; ++u) T[u] = v4d{0, 0, 0, 0};
+      for (int k0 = 0; k0 < nda; k0 += 16) {
+        double a[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) a[s] = an[s];
+#pragma unroll
+        for (int u = 0; u < NT; ++u)
+#pragma unroll
+          for (int s = 0; s < 4; ++s) d[u * 16 * 17 + dw + s * ds] = bn[u][s];
+        int kn = k0 + 16;
+        if (kn >= nda) {
+          kn = 0;
+          open_ab(min(t + 1, nt - 1));
+        }
+        load_ab(kn);
+        loads_first();                            // also: the patch is written before other lanes' values are read
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          if (s > 0 && k0 + 4 * s >= nda) break;
+#pragma unroll
+          for (int u = 0; u < NT; ++u) T[u] = mfma64(d[(u * 16 + 4 * s + mk) * 17 + mi], a[s], T[u]);
+        }
+        loads_first();                            // read before it is written again
+      }
+#pragma unroll
+      for (int u = 0; u < NT; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) tl[((t * 4 * NT + wave + 4 * u) * 4 + v) * 64 + lane] = sc * T[u][v];
+    }
+    open_c(0);
+    load_c(0);
+    loads_first();
+    __syncthreads();
+    for (int t = 0; t < nt; ++t) {
+      const int ndc = tm.ndc;
+      const double *T = tl + t * 4 * NT * 256 + lane;
+      for (int l0 = 0; l0 < ndc; l0 += 16) {
+        double cv[4][NT];
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+          for (int u = 0; u < NT; ++u) cv[v][u] = cn[v][u];
+        int ln = l0 + 16;
+        if (ln >= ndc) {
+          ln = 0;
+          open_c(min(t + 1, nt - 1));
+        }
+        load_c(ln);
+        loads_first();
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          if (v > 0 && l0 + 4 * v >= ndc) break;
+          const double a = T[(l0 / 4 + v) * 64];
+#pragma unroll
+          for (int u = 0; u < NT; ++u) acc[u] = mfma64(a, cv[v][u], acc[u]);
+        }
+      }
+    }
+    __syncthreads();                              // T has been read
+  }
+  double *O = obase + (size_t)w * ostride + (size_t)g.out_slot * nxy + g.out_off;
+#pragma unroll
+  for (int u = 0; u < NT; ++u) {
+    const int j = 16 * (wave + 4 * u) + mi;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = i0 + 4 * v + mk;
+      if (i < g.nrow && j < g.ncol) O[i + (size_t)j * g.nrow] = acc[u][v];
     }
   }
 }
@@ -2256,8 +2496,6 @@ struct pnfam_gpu_ctx {
   int ngroups_q2s[2] = {0, 0}, ngroups_s2q[2] = {0, 0};
   size_t lds_q2s = 0, lds_s2q = 0;
   int strips = 1;   // 16-row strips of the largest output block
-  // triprod groups sorted by column tiles: [stage q2s/s2q][ri][nct] -> first group, count, strips
-  int tp_first[2][2][TP_MAXCT + 1] = {}, tp_count[2][2][TP_MAXCT + 1] = {}, tp_strips[2][2][TP_MAXCT + 1] = {};
   DevPtr d_pairs;   // rho0, kap0, rho1, kap1 pair lists
   int pair_off[4] = {0, 0, 0, 0}, pair_n[4] = {0, 0, 0, 0};
   DevPtr d_tiles, d_tiles2;
@@ -2325,6 +2563,8 @@ struct pnfam_gpu_ctx {
   // split-BF16 block triple products (mixed path): padded hi/lo copies of U/V
   bool tp_bf16 = true;          // PNFAM_GPU_MIX_TRIPROD = bf16 | fp64
   bool tp_ready = false;
+  bool tp64_ok = true;          // the terms' A and C are whole blocks (FP64 matrix-core products)
+  DevPtr tp_cm64, tp_rm64;      // padded FP64 copies of U/V for them
   std::vector<int4> tp_blocks;  // (fp64 offset, padded offset, d, P) per block
   long tp_mstride = 0;
   DevPtr tp_rmh, tp_rml, tp_cmh, tp_cml, d_tp_blocks;
@@ -2501,57 +2741,8 @@ std::vector<int4> pair_list(const BlockMap &m) {
   return v;
 }
 
-// Orders a stage's groups by their number of 16-column tiles and records, per
-// tile count, the first group, the count and the 16-row strips of the tallest.
-void sort_groups_by_tiles(pnfam_gpu_ctx *h, int stage, int ri, std::vector<Group> &groups) {
-  auto nct = [](const Group &g) { return (g.ncol + 15) / 16; };
-  std::stable_sort(groups.begin(), groups.end(), [&](const Group &a, const Group &b) { return nct(a) < nct(b); });
-  for (int c = 0; c <= TP_MAXCT; ++c) { h->tp_first[stage][ri][c] = 0; h->tp_count[stage][ri][c] = 0; h->tp_strips[stage][ri][c] = 0; }
-  for (size_t i = 0; i < groups.size(); ++i) {
-    const int c = nct(groups[i]);
-    if (h->tp_count[stage][ri][c] == 0) h->tp_first[stage][ri][c] = (int)i;
-    h->tp_count[stage][ri][c]++;
-    h->tp_strips[stage][ri][c] = std::max(h->tp_strips[stage][ri][c], (groups[i].nrow + 15) / 16);
-  }
-}
-
-// One launch per tile count present in the stage.
-int launch_triprod(pnfam_gpu_ctx *h, int stage, int ri, const Group *groups, const Term *terms, const double *bbase,
-                   long bstride, double *obase, long ostride, int na, const int *act) {
-  const double *m0 = h->d_U[0].as<double>(), *m1 = h->d_U[1].as<double>(), *m2 = h->d_U[2].as<double>(),
-               *m3 = h->d_U[3].as<double>();
-  const bool merge = na <= TP_MERGE_N;
-  int cmax = 0, smax = 0, ntot = 0;
-  for (int c = 1; c <= TP_MAXCT; ++c)
-    if (h->tp_count[stage][ri][c]) { cmax = c; smax = std::max(smax, h->tp_strips[stage][ri][c]); ntot += h->tp_count[stage][ri][c]; }
-  for (int c = merge ? cmax : 1; c <= TP_MAXCT && c >= 1; ++c) {
-    const int n = merge ? ntot : h->tp_count[stage][ri][c];
-    if (!n) continue;
-    const dim3 grid(n, na, merge ? smax : h->tp_strips[stage][ri][c]);
-    const Group *g = groups + (merge ? 0 : h->tp_first[stage][ri][c]);
-    note(h, "k_triprod_mfma", std::min(c, TP_MAXCT));
-#define TP_LAUNCH(NC)                                                                                      \
-  hipLaunchKernelGGL(k_triprod_mfma<NC>, grid, dim3(64), 0, h->stream, g, terms, m0, m1, m2, m3, bbase, bstride, \
-                     obase, ostride, act, h->nxy, h->skip_slot)
-    switch (c) {
-      case 1: TP_LAUNCH(1); break;
-      case 2: TP_LAUNCH(2); break;
-      case 3: TP_LAUNCH(3); break;
-      case 4: TP_LAUNCH(4); break;
-      case 5: TP_LAUNCH(5); break;
-      case 6: TP_LAUNCH(6); break;
-      case 7: TP_LAUNCH(7); break;
-      default: TP_LAUNCH(8); break;
-    }
-#undef TP_LAUNCH
-    if (merge) break;
-  }
-  HIP_TRY(hipGetLastError());
-  return 0;
-}
-
-// Padded layout of the resident block-diagonal matrices for the BF16 triple
-// products: block i (dimension d, FP64 offset sum d_j^2) at the padded offset
+// Padded layout of the resident block-diagonal matrices for the matrix-core
+// triple products (BF16 and FP64): block i (dimension d, FP64 offset sum d_j^2) at the padded offset
 // sum P_j^2, P = d rounded up to 32.
 void tp_layout(pnfam_gpu_ctx *h) {
   h->tp_blocks.clear();
@@ -2645,8 +2836,7 @@ int tp_prepare(pnfam_gpu_ctx *h) {
   if (h->tp_ready) return 0;
   const size_t n = 4 * (size_t)h->tp_mstride * 2;
   int e;
-  if ((e = h->tp_rmh.alloc(n)) || (e = h->tp_rml.alloc(n)) || (e = h->tp_cmh.alloc(n)) || (e = h->tp_cml.alloc(n)) ||
-      (e = upload(h->d_tp_blocks, h->tp_blocks.data(), h->tp_blocks.size() * sizeof(int4), h->stream)))
+  if ((e = h->tp_rmh.alloc(n)) || (e = h->tp_rml.alloc(n)) || (e = h->tp_cmh.alloc(n)) || (e = h->tp_cml.alloc(n)))
     return e;
   for (int m = 0; m < 4; ++m) {
     const size_t o = (size_t)m * h->tp_mstride;
@@ -2657,6 +2847,54 @@ int tp_prepare(pnfam_gpu_ctx *h) {
   }
   HIP_TRY(hipGetLastError());
   h->tp_ready = true;
+  return 0;
+}
+
+// FP64 triple products of a stage, both term sets (re and im): one launch per
+// tile count present, or up to TP_SPLIT_N points one launch of k_triprod_split for
+// all of them (beyond that the groups alone fill the device; N_sh = 16, 4 points:
+// at 4 points 129 us, as much as the launches per count).
+int launch_triprod(pnfam_gpu_ctx *h, int stage, const double *bbase, long bstride, double *obase, long ostride, int na,
+                   const int *act) {
+  const Tp64 M{h->tp_cm64.as<double>(), h->tp_rm64.as<double>(), h->tp_mstride};
+  const Term *terms = h->d_tpa_terms[stage].as<Term>();
+  const Group *groups = h->d_tpa_groups[stage].as<Group>();
+  const bool split = na <= TP_SPLIT_N;
+  int cmax = 0, smax = 0, ntot = 0;
+  for (int c = 1; c <= TP_MAXCT; ++c)
+    if (h->tpa_count[stage][c]) { cmax = c; smax = std::max(smax, h->tpa_strips[stage][c]); ntot += h->tpa_count[stage][c]; }
+  for (int c = split ? cmax : 1; c <= TP_MAXCT && c >= 1; ++c) {
+    const int n = split ? ntot : h->tpa_count[stage][c];
+    if (!n) continue;
+    const int ns = split ? smax : h->tpa_strips[stage][c];
+    // four strips of a group to a workgroup, or two where that leaves fewer waves idle
+    const int nw = split || (ns + 1) % 4 < 2 ? 4 : 2, nz = split ? ns : (ns + nw - 1) / nw;
+    const dim3 grid(n, na, nz), block(64 * nw);
+    const Group *g = groups + (split ? 0 : h->tpa_first[stage][c]);
+    note(h, "k_triprod_mfma", std::min(c, TP_MAXCT));
+#define TP_GO(K) \
+  hipLaunchKernelGGL(K, grid, block, 0, h->stream, g, terms, M, bbase, bstride, obase, ostride, act, h->nxy, h->skip_slot)
+#define TP_LAUNCH(NC)                                      \
+  do {                                                     \
+    if (split) TP_GO(k_triprod_split<NC>);                 \
+    else if (nw == 4) TP_GO((k_triprod_mfma<NC, 4>));      \
+    else TP_GO((k_triprod_mfma<NC, 2>));                   \
+  } while (0)
+    switch (c) {
+      case 1: TP_LAUNCH(1); break;
+      case 2: TP_LAUNCH(2); break;
+      case 3: TP_LAUNCH(3); break;
+      case 4: TP_LAUNCH(4); break;
+      case 5: TP_LAUNCH(5); break;
+      case 6: TP_LAUNCH(6); break;
+      case 7: TP_LAUNCH(7); break;
+      default: TP_LAUNCH(8); break;
+    }
+#undef TP_LAUNCH
+#undef TP_GO
+    if (split) break;
+  }
+  HIP_TRY(hipGetLastError());
   return 0;
 }
 
@@ -2800,14 +3038,10 @@ int stage_qp2sp(pnfam_gpu_ctx *h, const double *vin, int na, const int *act, boo
                        h->skip_slot); }
   Prof pr(h, K_TRIPROD_Q2S, na);
   if (lowp) return launch_triprod_bf16(h, 0, vin, 4 * nxy, h->d_rsp.as<double>(), 8 * nxy, na, act, n3);
+  if (!h->basic_kernels && h->tp64_ok)
+    return launch_triprod(h, 0, vin, 4 * nxy, h->d_rsp.as<double>(), 8 * nxy, na, act);
   for (int ri = 0; ri < 2; ++ri) {
     if (!h->ngroups_q2s[ri]) continue;
-    if (!h->basic_kernels) {
-      if (int e = launch_triprod(h, 0, ri, h->d_groups_q2s[ri].as<Group>(), h->d_terms_q2s[ri].as<Term>(), vin, 4 * nxy,
-                                 h->d_rsp.as<double>(), 8 * nxy, na, act))
-        return e;
-      continue;
-    }
     hipLaunchKernelGGL(k_triprod, dim3(h->ngroups_q2s[ri], na), dim3(256), h->lds_q2s, h->stream,
                        h->d_groups_q2s[ri].as<Group>(), h->d_terms_q2s[ri].as<Term>(), h->d_U[0].as<double>(),
                        h->d_U[1].as<double>(), h->d_U[2].as<double>(), h->d_U[3].as<double>(), vin, 4 * nxy, 4,
@@ -3982,14 +4216,10 @@ int stage_sp2qp(pnfam_gpu_ctx *h, int na, const int *act, bool lowp = false, int
                        h->skip_slot); }
   Prof pr(h, K_TRIPROD_S2Q, na);
   if (lowp) return launch_triprod_bf16(h, 1, h->d_hsp.as<double>(), 8 * nxy, h->d_hqp.as<double>(), 4 * nxy, na, act, n3);
+  if (!h->basic_kernels && h->tp64_ok)
+    return launch_triprod(h, 1, h->d_hsp.as<double>(), 8 * nxy, h->d_hqp.as<double>(), 4 * nxy, na, act);
   for (int ri = 0; ri < 2; ++ri) {
     if (!h->ngroups_s2q[ri]) continue;
-    if (!h->basic_kernels) {
-      if (int e = launch_triprod(h, 1, ri, h->d_groups_s2q[ri].as<Group>(), h->d_terms_s2q[ri].as<Term>(),
-                                 h->d_hsp.as<double>(), 8 * nxy, h->d_hqp.as<double>(), 4 * nxy, na, act))
-        return e;
-      continue;
-    }
     hipLaunchKernelGGL(k_triprod, dim3(h->ngroups_s2q[ri], na), dim3(256), h->lds_s2q, h->stream,
                        h->d_groups_s2q[ri].as<Group>(), h->d_terms_s2q[ri].as<Term>(), h->d_U[0].as<double>(),
                        h->d_U[1].as<double>(), h->d_U[2].as<double>(), h->d_U[3].as<double>(), h->d_hsp.as<double>(),
@@ -4164,6 +4394,16 @@ int pnfam_gpu_create(const pnfam_gpu_basis *b, pnfam_gpu_ctx **out) {
       (e = upload(h->d_ns, h->ns.data(), (size_t)b->dqp * 4, h->stream)))
     return e;
   HIP_TRY(hipStreamSynchronize(h->stream));
+  // padded copies of U and V for the FP64 triple products
+  if ((e = h->tp_cm64.alloc(4 * (size_t)h->tp_mstride * 8)) || (e = h->tp_rm64.alloc(4 * (size_t)h->tp_mstride * 8)) ||
+      (e = upload(h->d_tp_blocks, h->tp_blocks.data(), h->tp_blocks.size() * sizeof(int4), h->stream)))
+    return e;
+  for (int m = 0; m < 4; ++m)
+    hipLaunchKernelGGL(k_tp_pack, dim3(16, (unsigned)h->tp_blocks.size()), dim3(256), 0, h->stream,
+                       h->d_U[m].as<double>(), h->d_tp_blocks.as<int4>(),
+                       h->tp_cm64.as<double>() + (size_t)m * h->tp_mstride,
+                       h->tp_rm64.as<double>() + (size_t)m * h->tp_mstride);
+  HIP_TRY(hipGetLastError());
   if ((e = sep_prepare(h.get(), b))) return e;
   *out = h.release();
   return 0;
@@ -4183,6 +4423,7 @@ int pnfam_gpu_set_operator(pnfam_gpu_ctx *h, int32_t beta_minus, const int32_t *
   }
   h->have_op = false;
   h->mix_ready = false;
+  h->tp64_ok = true;
   h->bminus = beta_minus != 0;
   const std::vector<int> &db = h->db;
   std::vector<int> diag(nb), tr(nb);
@@ -4256,9 +4497,8 @@ int pnfam_gpu_set_operator(pnfam_gpu_ctx *h, int32_t beta_minus, const int32_t *
     h->lds_q2s = std::max(h->lds_q2s, lds);
     if (ri == 0) h->flops_q2s = 0;
     for (auto &t : terms) h->flops_q2s += 2.0 * t.nda * t.nda * t.ndc + 2.0 * t.nda * t.ndc * t.ndc;
-    sort_groups_by_tiles(h, 0, ri, groups);
     tp_patch_terms(h, terms);
-    if (!tp_terms_ok(terms)) h->tp_bf16 = false;   // A or C not whole blocks: FP64 products only
+    if (!tp_terms_ok(terms)) h->tp_bf16 = h->tp64_ok = false;   // A or C not whole blocks: the plain FP64 products only
     int e;
     if (ri == 0) { h->tpa_terms_h[0].clear(); h->tpa_groups_h[0].clear(); h->tpa_toff_h[0].clear(); h->tpa_jobs_h[0].clear(); }
     h->tp_L[0] = tp_b_layout(h, 0, terms, groups, ri == 0 ? 0 : h->tp_L[0]);
@@ -4297,9 +4537,8 @@ int pnfam_gpu_set_operator(pnfam_gpu_ctx *h, int32_t beta_minus, const int32_t *
     h->lds_s2q = std::max(h->lds_s2q, lds);
     if (ri == 0) h->flops_s2q = 0;
     for (auto &t : terms) h->flops_s2q += 2.0 * t.nda * t.nda * t.ndc + 2.0 * t.nda * t.ndc * t.ndc;
-    sort_groups_by_tiles(h, 1, ri, groups);
     tp_patch_terms(h, terms);
-    if (!tp_terms_ok(terms)) h->tp_bf16 = false;   // A or C not whole blocks: FP64 products only
+    if (!tp_terms_ok(terms)) h->tp_bf16 = h->tp64_ok = false;   // A or C not whole blocks: the plain FP64 products only
     int e;
     if (ri == 0) { h->tpa_terms_h[1].clear(); h->tpa_groups_h[1].clear(); h->tpa_toff_h[1].clear(); h->tpa_jobs_h[1].clear(); }
     h->tp_L[1] = tp_b_layout(h, 1, terms, groups, ri == 0 ? 0 : h->tp_L[1]);
