@@ -2624,7 +2624,7 @@ struct pnfam_gpu_ctx {
   DevPtr d_sep_f, d_sep_fz;
   DevPtr d_sep_keys, d_sep_tabs, d_sep_djobs, d_sep_pjobs;
   DevPtr d_sep_slots[2], d_sep_elems[2];         // density, projection
-  int sep_nslot[2] = {0, 0}, sep_ndjob = 0, sep_npjob[2] = {0, 0}, sep_pjob0[2] = {0, 0};
+  int sep_nslot[2] = {0, 0}, sep_ndjob = 0, sep_nwork = 0, sep_npjob[2] = {0, 0}, sep_pjob0[2] = {0, 0};
   int sep_ct[2] = {1, 1}, sep_ncg[2] = {1, 1};   // density, projection: column tiles per wave, column groups
   SepAcc sep_acc{};
   long sep_zstride = 0, sep_ystride = 0, sep_arows = 0;
@@ -3376,8 +3376,10 @@ int sep_build(pnfam_gpu_ctx *h) {
   }
   std::vector<SepSlot> slots[2];
   std::vector<int4> elems[2];
-  std::vector<SepDJob> djobs;
-  std::vector<SepPJob> pjobs[2];
+  struct Bundle { int first, count; };   // slots with the same columns
+  std::vector<Bundle> bundles[2];
+  std::vector<std::vector<SepDJob>> dgroups;
+  std::vector<std::vector<SepPJob>> pgroups[2];
   long zoff = 0, yoff = 0, arow = 0;
   h->sep_flops_d = h->sep_flops_p = 0;
   // the slots of one class with their elements; each slot takes `ld` doubles from `at` on
@@ -3397,7 +3399,14 @@ int sep_build(pnfam_gpu_ctx *h) {
             }
         }
     }
-    for (size_t s = 0; s < el.size(); ++s) {
+    // in the order of the columns' function, one bundle for each
+    std::vector<int> order(el.size());
+    std::iota(order.begin(), order.end(), 0);
+    std::stable_sort(order.begin(), order.end(), [&](int a, int c) { return T.keys[a].second < T.keys[c].second; });
+    for (size_t k = 0; k < order.size(); ++k) {
+      const int s = order[k];
+      if (k == 0 || T.keys[s].second != T.keys[order[k - 1]].second) bundles[side].push_back({(int)slots[side].size(), 0});
+      ++bundles[side].back().count;
       slots[side].push_back({(int)elems[side].size(), (int)el[s].size(), mat, (int)(at + (long)s * ld)});
       elems[side].insert(elems[side].end(), el[s].begin(), el[s].end());
     }
@@ -3411,10 +3420,15 @@ int sep_build(pnfam_gpu_ctx *h) {
       put_slots(0, q, T, *dm[mat], zoff, (long)nt * W);
       h->sep_acc.row[q] = n ? (int)arow : -1;
       for (int t = 0; t < nt && n; ++t) {
-        const int r0 = sep_row0(kind, same, t, nr), r1 = sep_row0(kind, same, t + 1, nr);
-        for (int r = r0; r < r1; r += 64)
-          djobs.push_back({tb + T.rd, n, ld, r, std::min(4, (r1 - r) / 16), (int)(zoff + (long)t * W), nt * W,
-                           (int)arow + r, 0});
+        const int r0 = sep_row0(kind, same, t, nr), r1 = sep_row0(kind, same, t + 1, nr), tiles = (r1 - r0) / 16;
+        const int nw = (tiles + 3) / 4;             // waves: at most four row tiles each, evenly
+        std::vector<SepDJob> g;                     // one group: they read the same Z rows
+        for (int k = 0, r = r0; k < nw; ++k) {
+          const int q = tiles / nw + (k < tiles % nw ? 1 : 0);
+          g.push_back({(int64_t)T.rd, n, ld, r, q, (int)(zoff + (long)t * W), nt * W, (int)arow + r, 0});
+          r += 16 * q;
+        }
+        dgroups.push_back(g);
         h->sep_flops_d += 2.0 * n * sep_rows(kind, same, t) * nr * W;
       }
       zoff += (long)n * nt * W;
@@ -3426,12 +3440,19 @@ int sep_build(pnfam_gpu_ctx *h) {
       put_slots(1, q, T, *pm[mat], yoff, (long)nt * W8);
       for (int t = 0; t < nt && n; ++t) {
         h->sep_flops_p += 2.0 * n * sep_terms(kind, same, t) * nr * W;
+        uint64_t fields = 0;
+        for (int c = sep_terms(kind, same, t) - 1; c >= 0; --c) fields = fields << 7 | (uint64_t)sep_field(kind, t, c, sa, sb);
         for (int v = 0; v < 2; ++v) {
           const int rt = v ? 4 : 1;
-          for (int s = 0; s < ld; s += 16 * rt)
-            pjobs[v].push_back({tb + T.rp + (size_t)sep_k0(kind, same, t, nr4) * ld, ld, n, s,
-                                std::min(rt, (ld - s) / 16), sep_terms(kind, same, t), t, kind, sa, sb, mat >> 1,
-                                (int)(yoff + (long)t * W8), nt * W8});
+          std::vector<SepPJob> g;                   // one group: they read the same fields
+          for (int s = 0; s < ld; s += 16 * rt) {
+            if ((int)g.size() == SEP_PRUN) { pgroups[v].push_back(g); g.clear(); }
+            g.push_back({(int64_t)(T.rp + (size_t)sep_k0(kind, same, t, nr4) * ld), fields, ld, n, s,
+                         std::min(rt, (ld - s) / 16), sep_terms(kind, same, t), mat >> 1, (int)(yoff + (long)t * W8),
+                         nt * W8});
+          }
+          g.resize(SEP_PRUN, SepPJob{});
+          pgroups[v].push_back(g);
         }
       }
       yoff += (long)n * nt * W8;
@@ -3441,14 +3462,56 @@ int sep_build(pnfam_gpu_ctx *h) {
     h->sep_flops_p += (kind ? 4.0 : 20.0) * nz * (double)pm[mat]->nelem(h->db) / 4;
     if (zoff > (1L << 30) || yoff > (1L << 30)) return 0;   // offsets are 32-bit: such a basis keeps the other kernels
   }
-  // longest first, so that the last workgroups of a launch are short ones
-  std::stable_sort(djobs.begin(), djobs.end(), [](const SepDJob &a, const SepDJob &b) { return a.n * a.nrt > b.n * b.nrt; });
-  for (auto &v : pjobs)
-    std::stable_sort(v.begin(), v.end(), [](const SepPJob &a, const SepPJob &b) { return a.nc * a.nst > b.nc * b.nst; });
-  for (auto &v : slots)
-    std::stable_sort(v.begin(), v.end(), [](const SepSlot &a, const SepSlot &b) {
-      return (a.mat & 1) != (b.mat & 1) ? (a.mat & 1) < (b.mat & 1) : a.count > b.count;
-    });
+  // the job groups go to the XCD with the least work so far, the costliest group
+  // first; lists of unequal length end in empty jobs
+  auto deal = [](auto &groups, auto cost, auto &all) {
+    auto sum = [&](const auto &g) {
+      long c = 0;
+      for (auto &j : g) c += cost(j);
+      return c;
+    };
+    std::stable_sort(groups.begin(), groups.end(), [&](const auto &a, const auto &b) { return sum(a) > sum(b); });
+    typename std::remove_reference<decltype(groups[0])>::type list[8];
+    long load[8] = {};
+    for (auto &g : groups) {
+      const int x = (int)(std::min_element(load, load + 8) - load);
+      load[x] += sum(g);
+      list[x].insert(list[x].end(), g.begin(), g.end());
+    }
+    size_t len = 0;
+    for (auto &l : list) len = std::max(len, l.size());
+    all.assign(8 * len, typename std::remove_reference<decltype(all[0])>::type{});
+    for (int x = 0; x < 8; ++x) std::copy(list[x].begin(), list[x].end(), all.begin() + x * len);
+  };
+  std::vector<SepDJob> djobs;
+  std::vector<SepPJob> pjobs[2];
+  deal(dgroups, [](const SepDJob &j) { return (long)j.n * j.nrt; }, djobs);
+  for (int v = 0; v < 2; ++v) deal(pgroups[v], [](const SepPJob &j) { return (long)j.nc * j.nst; }, pjobs[v]);
+  // the bundles dealt to the eight XCDs in turn, the costliest first; workgroup x
+  // (four slots) runs on XCD x % 8, lists of unequal length end in empty slots
+  for (int k = 0; k < 2; ++k) {
+    auto cost = [&](const Bundle &b) {
+      long c = 0;
+      for (int i = 0; i < b.count; ++i) {
+        const SepSlot &s = slots[k][b.first + i];
+        c += (long)(s.count + 16) * ((s.mat & 1) ? 1 : 4);
+      }
+      return c;
+    };
+    std::stable_sort(bundles[k].begin(), bundles[k].end(), [&](const Bundle &a, const Bundle &b) { return cost(a) > cost(b); });
+    std::vector<SepSlot> xcd[8];
+    for (size_t i = 0; i < bundles[k].size(); ++i) {
+      auto &x = xcd[i % 8];
+      const auto first = slots[k].begin() + bundles[k][i].first;
+      x.insert(x.end(), first, first + bundles[k][i].count);
+    }
+    size_t len = 0;
+    for (auto &x : xcd) len = std::max(len, (x.size() + 3) / 4 * 4);
+    std::vector<SepSlot> all(8 * len, SepSlot{0, 0, 0, 0});
+    for (int x = 0; x < 8; ++x)
+      for (size_t i = 0; i < xcd[x].size(); ++i) all[((i / 4) * 8 + x) * 4 + i % 4] = xcd[x][i];
+    slots[k].swap(all);
+  }
   std::vector<SepPJob> pj(pjobs[0]);
   pj.insert(pj.end(), pjobs[1].begin(), pjobs[1].end());
   for (int k = 0; k < 2; ++k) {
@@ -3462,6 +3525,7 @@ int sep_build(pnfam_gpu_ctx *h) {
     return e;
   HIP_TRY(hipStreamSynchronize(h->stream));   // pageable sources
   h->sep_ndjob = (int)djobs.size();
+  h->sep_nwork = (int)std::count_if(djobs.begin(), djobs.end(), [](const SepDJob &j) { return j.n > 0; });
   for (int v = 0; v < 2; ++v) {
     h->sep_pjob0[v] = v ? (int)pjobs[0].size() : 0;
     h->sep_npjob[v] = (int)pjobs[v].size();
@@ -3478,14 +3542,14 @@ bool sep_active(const pnfam_gpu_ctx *h) {
 // Points a pass of the separable stage takes at once, and the splits of its
 // density contraction: with few points the slots are split so that about 2 048
 // waves run.
-constexpr size_t SEP_CHUNK_BYTES = size_t(1) << 30;
+constexpr size_t SEP_CHUNK_BYTES = size_t(4) << 30;
 int sep_chunk(const pnfam_gpu_ctx *h, int na) {
   const size_t per = (size_t)std::max(h->sep_zstride, h->sep_ystride) * 8;
   return (int)std::max<size_t>(1, std::min<size_t>((size_t)na, SEP_CHUNK_BYTES / std::max<size_t>(1, per)));
 }
 int sep_split(const pnfam_gpu_ctx *h, int nc, bool split) {
   if (!split) return 1;
-  const long waves = (long)h->sep_ndjob * h->sep_ncg[0] * nc;
+  const long waves = (long)h->sep_nwork * h->sep_ncg[0] * nc;
   return (int)std::max<long>(1, std::min<long>(16, 2048 / std::max<long>(1, waves)));
 }
 
@@ -3504,7 +3568,7 @@ int sep_workspace(pnfam_gpu_ctx *h, int na) {
 int stage_hamiltonian_sep(pnfam_gpu_ctx *h, int na, const int *act, const GridBufs &gb) {
   SepArgs A{};
   A.nz = h->sep_nz; A.nr = h->sep_nr; A.dqp = h->dqp; A.nxy = h->nxy;
-  A.nzp = sep_pad8(A.nz); A.fz = h->d_sep_fz.as<double>();
+  A.nzp = sep_pad8(A.nz); A.fz = h->d_sep_fz.as<double>(); A.tab = h->d_sep_tabs.as<double>();
   A.rsp = gb.rsp; A.dens = gb.dens; A.flds = gb.flds; A.hsp = gb.hsp; A.wdcori = h->d_wdcori.as<double>();
   A.slot_of[0] = 0; A.slot_of[1] = 1; A.slot_of[2] = gb.rho1; A.slot_of[3] = gb.kap1;
   A.zy = h->d_sep_zy.as<double>(); A.zstride = h->sep_zstride; A.ystride = h->sep_ystride;
@@ -3520,16 +3584,16 @@ int stage_hamiltonian_sep(pnfam_gpu_ctx *h, int na, const int *act, const GridBu
       const int ns = sep_split(h, nc, gb.split);
       note(h, "k_sep_dens", h->sep_ct[0], ns);
       const int zt = (h->sep_nz + 15) / 16, zg = (zt + 2) / 3;
-      const dim3 zgrid((h->sep_nslot[0] + 3) / 4, (nc + 7) / 8, zg);
+      const dim3 zgrid(h->sep_nslot[0] / 4, (nc + 7) / 8, zg);
       const SepSlot *sl = h->d_sep_slots[0].as<SepSlot>();
       const int4 *el = h->d_sep_elems[0].as<int4>();
       switch ((zt + zg - 1) / zg) {
-        case 1: hipLaunchKernelGGL(k_sep_z<1>, zgrid, dim3(256), 0, h->stream, A, sl, el, h->sep_nslot[0]); break;
-        case 2: hipLaunchKernelGGL(k_sep_z<2>, zgrid, dim3(256), 0, h->stream, A, sl, el, h->sep_nslot[0]); break;
-        default: hipLaunchKernelGGL(k_sep_z<3>, zgrid, dim3(256), 0, h->stream, A, sl, el, h->sep_nslot[0]); break;
+        case 1: hipLaunchKernelGGL(k_sep_z<1>, zgrid, dim3(256), 0, h->stream, A, sl, el); break;
+        case 2: hipLaunchKernelGGL(k_sep_z<2>, zgrid, dim3(256), 0, h->stream, A, sl, el); break;
+        default: hipLaunchKernelGGL(k_sep_z<3>, zgrid, dim3(256), 0, h->stream, A, sl, el); break;
       }
-      const dim3 grid(h->sep_ndjob, nc, h->sep_ncg[0] * ns);
-#define SEP_D(CT) hipLaunchKernelGGL(k_sep_dens<CT>, grid, dim3(64), 0, h->stream, A, h->d_sep_djobs.as<SepDJob>(), h->sep_ncg[0], ns)
+      const dim3 grid(h->sep_ndjob * nc, h->sep_ncg[0] * ns);
+#define SEP_D(CT) hipLaunchKernelGGL(k_sep_dens<CT>, grid, dim3(64), 0, h->stream, A, h->d_sep_djobs.as<SepDJob>(), h->sep_ndjob, h->sep_ncg[0], ns)
       switch (h->sep_ct[0]) {
         case 1: SEP_D(1); break;
         case 2: SEP_D(2); break;
@@ -3552,12 +3616,13 @@ int stage_hamiltonian_sep(pnfam_gpu_ctx *h, int na, const int *act, const GridBu
     { Prof pr(h, K_PROJECT, nc);
       const int v = nc >= 8 ? 1 : 0;   // four slot tiles per wave from eight points, one below
       note(h, "k_sep_proj", h->sep_ct[1], v ? 4 : 1);
-      const dim3 grid(h->sep_npjob[v], nc, h->sep_ncg[1]);
+      const dim3 grid(h->sep_npjob[v] * nc, h->sep_ncg[1]);
+      const int np = h->sep_npjob[v];
       const SepPJob *pj = h->d_sep_pjobs.as<SepPJob>() + h->sep_pjob0[v];
 #define SEP_P(CT)                                                                                    \
   do {                                                                                               \
-    if (v) hipLaunchKernelGGL((k_sep_proj<CT, 4>), grid, dim3(64), 0, h->stream, A, pj);             \
-    else hipLaunchKernelGGL((k_sep_proj<CT, 1>), grid, dim3(64), 0, h->stream, A, pj);               \
+    if (v) hipLaunchKernelGGL((k_sep_proj<CT, 4>), grid, dim3(64), 0, h->stream, A, pj, np);        \
+    else hipLaunchKernelGGL((k_sep_proj<CT, 1>), grid, dim3(64), 0, h->stream, A, pj, np);             \
   } while (0)
       switch (h->sep_ct[1]) {
         case 1: SEP_P(1); break;
@@ -3567,8 +3632,12 @@ int stage_hamiltonian_sep(pnfam_gpu_ctx *h, int na, const int *act, const GridBu
         default: SEP_P(5); break;
       }
 #undef SEP_P
-      hipLaunchKernelGGL(k_sep_expand, dim3((h->sep_nslot[1] + 3) / 4, (nc + 7) / 8), dim3(256), 0, h->stream, A,
-                         h->d_sep_slots[1].as<SepSlot>(), h->d_sep_elems[1].as<int4>(), h->sep_nslot[1]);
+      const SepSlot *sl = h->d_sep_slots[1].as<SepSlot>();
+      const int4 *el = h->d_sep_elems[1].as<int4>();
+      if (nc > 8)
+        hipLaunchKernelGGL(k_sep_expand<2>, dim3(h->sep_nslot[1] / 4, (nc + 15) / 16), dim3(256), 0, h->stream, A, sl, el);
+      else
+        hipLaunchKernelGGL(k_sep_expand<1>, dim3(h->sep_nslot[1] / 4, 1), dim3(256), 0, h->stream, A, sl, el);
     }
   }
   HIP_TRY(hipGetLastError());

@@ -203,7 +203,7 @@ __host__ __device__ inline int sep_k0(int kind, bool same, int t, int nr4) {
   return o;
 }
 // field component (index of the 104) of term c of axial pair t
-__device__ inline int sep_field(int kind, int t, int c, int sa, int sb) {
+inline int sep_field(int kind, int t, int c, int sa, int sb) {
   if (kind) return 100 + (sb == 0 ? (sa == 0 ? 0 : 1) : (sa == 0 ? 2 : 3));
   int z, zp;
   if (t == 0) {   // 00, 01, 10, 02, 20, 11, 12, 04, 22
@@ -299,10 +299,13 @@ __global__ void k_sep_rtab(SepTab T, const double *__restrict__ ftab, int nr, in
 // ---- densities: axial contraction ----------------------------------------------
 // A slot's matrix elements: offset in the structure's storage, row and column state.
 struct SepSlot { int first, count, mat, zoff; };   // elements; offset of its Z rows (densities) or Y rows (projection)
+// The slots of one structure, pair of spins and radial function of the columns
+// form a bundle: they read (write) rows of the same matrix columns.
 struct SepArgs {
   int nz, nr, dqp, nzp;       // nzp: nz padded to 8, the stride of the axial tables and of Y
   long nxy;
   const double *fz;           // [3][dqp][nzp]
+  const double *tab;          // tables of radial products
   const double *rsp;          // [w][8][nxy]
   int slot_of[4];             // rsp slots (pairs) of rho0, kap0, rho1, kap1
   double *zy;                 // per active point: Z, later Y
@@ -324,36 +327,40 @@ struct SepArgs {
 // leave rows of the matrix instructions empty, which costs less than the
 // scalar loads of a vector kernel did (one lane per axial point, rho through
 // scalar loads: 2.3 ms for 48 points of N_sh = 16, 75 us for one).
-template <int ZT>
-__global__ void __launch_bounds__(256) k_sep_z(SepArgs A, const SepSlot *__restrict__ slots,
-                                               const int4 *__restrict__ elems, int nslot) {
-  const int id = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
-  if (id >= nslot) return;
-  const SepSlot S = slots[id];
+// The prefetched loads are unconditional (clamped to the list) so that they stay
+// in flight across the products: a load under a branch is waited for at its end.
+template <int ZT, bool MEAN>
+__device__ inline void sep_z_slot(const SepArgs &A, const SepSlot S, const int4 *__restrict__ elems) {
+  constexpr int NX = MEAN ? 4 : 1;
   const int lane = threadIdx.x & 63, mi = lane & 15, mk = lane >> 4;
-  const bool mean = (S.mat & 1) == 0;
   const int y = min((int)blockIdx.y * 8 + (mi >> 1), A.na - 1);
   const double *__restrict__ rho = A.rsp + ((size_t)A.act[y] * 8 + 2 * A.slot_of[S.mat] + (mi & 1)) * A.nxy;
   const size_t xs = (size_t)A.dqp * A.nzp;
+  // rows this lane stores (row 4 v + mk of the product)
+  bool st[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int yo = blockIdx.y * 8 + 2 * v + (mk >> 1);
+    st[v] = yo < A.na && A.act[min(yo, A.na - 1)] != A.skip;
+  }
   int z[ZT];
 #pragma unroll
   for (int t = 0; t < ZT; ++t) z[t] = min((int)(blockIdx.z * ZT + t) * 16 + mi, A.nzp - 1);
-  v4d C[ZT][4];
+  v4d C[ZT][NX];
 #pragma unroll
   for (int t = 0; t < ZT; ++t)
 #pragma unroll
-    for (int k = 0; k < 4; ++k) C[t][k] = v4d{0, 0, 0, 0};
+    for (int k = 0; k < NX; ++k) C[t][k] = v4d{0, 0, 0, 0};
   const int4 *__restrict__ el = elems + S.first;
   auto load = [&](int4 r, double (&c)[ZT][4]) {
+    const double *fa = A.fz + (size_t)r.y * A.nzp, *fb = A.fz + (size_t)r.z * A.nzp;
 #pragma unroll
     for (int t = 0; t < ZT; ++t) {
-      c[t][0] = A.fz[(size_t)r.y * A.nzp + z[t]];
-      c[t][2] = A.fz[(size_t)r.z * A.nzp + z[t]];
-      if (mean) {
-        c[t][1] = A.fz[xs + (size_t)r.y * A.nzp + z[t]];
-        c[t][3] = A.fz[xs + (size_t)r.z * A.nzp + z[t]];
-      } else {
-        c[t][1] = c[t][3] = 0.0;
+      c[t][0] = fa[z[t]];
+      c[t][2] = fb[z[t]];
+      if (MEAN) {
+        c[t][1] = fa[xs + z[t]];
+        c[t][3] = fb[xs + z[t]];
       }
     }
   };
@@ -364,118 +371,148 @@ __global__ void __launch_bounds__(256) k_sep_z(SepArgs A, const SepSlot *__restr
   rn = el[min(4 + mk, n - 1)];
   for (int s = 0; s < n; s += 4) {
     const double v = s + mk < n ? vn : 0.0;
-    double c[ZT][4];
-#pragma unroll
-    for (int t = 0; t < ZT; ++t)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) c[t][k] = cn[t][k];
-    if (s + 4 < n) {
-      vn = rho[rn.x];
-      load(rn, cn);
-      rn = el[min(s + 8 + mk, n - 1)];
-    }
+    double X[ZT][NX];
 #pragma unroll
     for (int t = 0; t < ZT; ++t) {
-      C[t][0] = mfma64(v, c[t][0] * c[t][2], C[t][0]);
-      if (mean) {
-        C[t][1] = mfma64(v, c[t][0] * c[t][3], C[t][1]);
-        C[t][2] = mfma64(v, c[t][1] * c[t][2], C[t][2]);
-        C[t][3] = mfma64(v, c[t][1] * c[t][3], C[t][3]);
+      X[t][0] = cn[t][0] * cn[t][2];
+      if (MEAN) {
+        X[t][NX / 2 - 1] = cn[t][0] * cn[t][3];
+        X[t][NX / 2] = cn[t][1] * cn[t][2];
+        X[t][NX - 1] = cn[t][1] * cn[t][3];
       }
     }
+    vn = rho[rn.x];
+    load(rn, cn);
+    rn = el[min(s + 8 + mk, n - 1)];
+    loads_first();
+#pragma unroll
+    for (int k = 0; k < NX; ++k)
+#pragma unroll
+      for (int t = 0; t < ZT; ++t) C[t][k] = mfma64(v, X[t][k], C[t][k]);
   }
+  double *out = A.zy + (size_t)(blockIdx.y * 8 + (mk >> 1)) * A.zstride + S.zoff + (size_t)(mk & 1) * A.nz;
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
-    const int yo = blockIdx.y * 8 + 2 * v + (mk >> 1);     // row 4 v + mk of the product
-    if (yo >= A.na || A.act[yo] == A.skip) continue;
-    double *out = A.zy + (size_t)yo * A.zstride + S.zoff + (size_t)(mk & 1) * A.nz;
+    if (st[v])
 #pragma unroll
-    for (int t = 0; t < ZT; ++t) {
-      const int zt = (blockIdx.z * ZT + t) * 16 + mi;
-      if (zt < A.nz)
+      for (int t = 0; t < ZT; ++t) {
+        const int zt = (blockIdx.z * ZT + t) * 16 + mi;
+        if (zt < A.nz)
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-          if (k == 0 || mean) out[(size_t)(2 * k) * A.nz + zt] = C[t][k][v];
-    }
+          for (int k = 0; k < NX; ++k) out[(size_t)(2 * k) * A.nz + zt] = C[t][k][v];
+      }
+    out += 2 * A.zstride;
   }
+}
+
+// Four slots of a bundle per workgroup, one per wave; the host deals the bundles
+// to the XCDs (workgroup x runs on XCD x % 8), so that a bundle's lines are
+// fetched into one L2.
+template <int ZT>
+__global__ void __launch_bounds__(256) k_sep_z(SepArgs A, const SepSlot *__restrict__ slots,
+                                               const int4 *__restrict__ elems) {
+  const SepSlot S = slots[__builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)))];
+  if (S.count == 0) return;
+  if ((S.mat & 1) == 0) sep_z_slot<ZT, true>(A, S, elems);
+  else sep_z_slot<ZT, false>(A, S, elems);
 }
 
 // ---- densities: radial contraction ----------------------------------------------
 struct SepDJob {            // 16-row tiles of one axial pair of one (structure, spins)
-  const double *rd;         // table of the class
+  int64_t rd;               // offset of the class's table
   int n, ld;                // slots; rows per slot
-  int row, nrt;             // first table row, tiles (1..4)
+  int row, nrt;             // first table row, tiles (1..4; 0: an empty job)
   int zoff, zld;            // Z of the class's first slot at this axial pair; stride between slots
   int arow, pad;            // output row of the first tile
 };
+
+// The jobs of the two radial contractions: workgroup b runs on XCD b % 8 and takes
+// that XCD's jobs (list entries [x len, (x + 1) len), len = njob / 8), `run` jobs
+// at a time for every point: the tables of a run stay in the XCD's L2 while the
+// points pass by, and its jobs, which read the same operands of a point, run side
+// by side.
+__device__ inline int sep_job(int njob, int run, int na, int &y) {
+  const int x = blockIdx.x & 7, i = blockIdx.x >> 3, g = i / (run * na), r = i - g * run * na;
+  y = r / run;
+  return x * (njob >> 3) + g * run + r % run;
+}
+
+// One job with RT row tiles.  No branch in the loop (a job's tile count is a
+// template argument, the load after the last step repeats it), so that the loads
+// of a step stay in flight across the products of the one before.
+template <int CT, int RT>
+__device__ inline void sep_dens_job(const SepArgs &A, const SepDJob &J, int y, int ncg, int nsplit) {
+  const int lane = threadIdx.x, mi = lane & 15, mk = lane >> 4;
+  const int cg = blockIdx.y % ncg, spl = blockIdx.y / ncg;
+  const int W = 2 * A.nz;
+  const int nst = (J.n + 3) >> 2;
+  const int s0 = (int)((long)spl * nst / nsplit), s1 = (int)((long)(spl + 1) * nst / nsplit);
+  v4d C[RT][CT];
+#pragma unroll
+  for (int q = 0; q < RT; ++q)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) C[q][c] = v4d{0, 0, 0, 0};
+  if (s0 < s1) {
+    const double *__restrict__ R = A.tab + J.rd + J.row + mi;
+    const double *__restrict__ Z = A.zy + (size_t)y * A.zstride + J.zoff;
+    int col[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) col[c] = min((cg * CT + c) * 16 + mi, W - 1);
+    double an[RT], bn[CT];
+    auto load = [&](int s) {
+      const int p = 4 * s + mk;                    // table rows are zero past the last slot
+      const double *r = R + (size_t)p * J.ld, *z = Z + (size_t)min(p, J.n - 1) * J.zld;
+#pragma unroll
+      for (int q = 0; q < RT; ++q) an[q] = r[16 * q];
+#pragma unroll
+      for (int c = 0; c < CT; ++c) bn[c] = z[col[c]];
+    };
+    load(s0);
+    for (int s = s0; s < s1; ++s) {
+      double a[RT], b[CT];
+#pragma unroll
+      for (int q = 0; q < RT; ++q) a[q] = an[q];
+#pragma unroll
+      for (int c = 0; c < CT; ++c) b[c] = bn[c];
+      load(min(s + 1, s1 - 1));
+      loads_first();
+#pragma unroll
+      for (int q = 0; q < RT; ++q)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) C[q][c] = mfma64(a[q], b[c], C[q][c]);
+    }
+  }
+  double *out = A.acc + ((size_t)spl * A.na + y) * A.astride + (size_t)J.arow * W;
+#pragma unroll
+  for (int q = 0; q < RT; ++q)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      const int k = (cg * CT + c) * 16 + mi;
+      if (k < W)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) out[(size_t)(16 * q + 4 * v + mk) * W + k] = C[q][c][v];
+    }
+}
 
 // acc(row, (ri, z)) = sum_p R[p][row] Z_t[p][(ri, z)] on v_mfma_f64_16x16x4:
 // up to 4 row tiles by CT column tiles per wave, four slots per step, the
 // operands of the next step in flight during the products of this one.  One
 // wave's 20 products of a step (1 280 cycles at 40 points) hide its 9 operand
-// loads; the tables are shared by all frequencies and stay in L2.  With few
-// points the slots are split (blockIdx.z), the parts added in order by
-// k_sep_sum.
+// loads; an XCD reads its own part of the tables only.  With few points the slots
+// are split (blockIdx.y), the parts added in order by k_sep_sum.
 template <int CT>
-__global__ void __launch_bounds__(64) k_sep_dens(SepArgs A, const SepDJob *__restrict__ jobs, int ncg, int nsplit) {
-  const int w = A.act[blockIdx.y];
-  if (w == A.skip) return;
-  const SepDJob J = jobs[blockIdx.x];
-  const int lane = threadIdx.x, mi = lane & 15, mk = lane >> 4;
-  const int cg = blockIdx.z % ncg, spl = blockIdx.z / ncg;
-  const int W = 2 * A.nz;
-  const int nst = (J.n + 3) >> 2;
-  const int s0 = (int)((long)spl * nst / nsplit), s1 = (int)((long)(spl + 1) * nst / nsplit);
-  v4d C[4][CT];
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-#pragma unroll
-    for (int c = 0; c < CT; ++c) C[q][c] = v4d{0, 0, 0, 0};
-  const double *__restrict__ R = J.rd + J.row + mi;
-  const double *__restrict__ Z = A.zy + (size_t)blockIdx.y * A.zstride + J.zoff;
-  int col[CT];
-#pragma unroll
-  for (int c = 0; c < CT; ++c) {
-    const int k = (cg * CT + c) * 16 + mi;
-    col[c] = k < W ? k : W - 1;
+__global__ void __launch_bounds__(64, 2) k_sep_dens(SepArgs A, const SepDJob *__restrict__ jobs, int njob, int ncg,
+                                                    int nsplit) {
+  int y;
+  const SepDJob J = jobs[sep_job(njob, njob >> 3, A.na, y)];
+  if (A.act[y] == A.skip) return;
+  switch (J.nrt) {
+    case 1: sep_dens_job<CT, 1>(A, J, y, ncg, nsplit); break;
+    case 2: sep_dens_job<CT, 2>(A, J, y, ncg, nsplit); break;
+    case 3: sep_dens_job<CT, 3>(A, J, y, ncg, nsplit); break;
+    case 4: sep_dens_job<CT, 4>(A, J, y, ncg, nsplit); break;
+    default: break;
   }
-  auto load = [&](int s, double (&a)[4], double (&b)[CT]) {
-    const int p = 4 * s + mk;                    // table rows are zero past the last slot
-    const double *r = R + (size_t)p * J.ld;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) a[q] = q < J.nrt ? r[16 * q] : 0.0;
-    const double *z = Z + (size_t)min(p, J.n - 1) * J.zld;
-#pragma unroll
-    for (int c = 0; c < CT; ++c) b[c] = z[col[c]];
-  };
-  if (s0 < s1) {
-    double an[4], bn[CT];
-    load(s0, an, bn);
-    for (int s = s0; s < s1; ++s) {
-      double a[4], b[CT];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) a[q] = an[q];
-#pragma unroll
-      for (int c = 0; c < CT; ++c) b[c] = bn[c];
-      if (s + 1 < s1) load(s + 1, an, bn);
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        if (q < J.nrt)
-#pragma unroll
-          for (int c = 0; c < CT; ++c) C[q][c] = mfma64(a[q], b[c], C[q][c]);
-    }
-  }
-  double *out = A.acc + ((size_t)spl * A.na + blockIdx.y) * A.astride + (size_t)J.arow * W;
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    if (q < J.nrt)
-#pragma unroll
-      for (int c = 0; c < CT; ++c) {
-        const int k = (cg * CT + c) * 16 + mi;
-        if (k < W)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) out[(size_t)(16 * q + 4 * v + mk) * W + k] = C[q][c][v];
-      }
 }
 
 // acc of split 0 += those of the other splits, in order
@@ -551,24 +588,19 @@ __global__ void __launch_bounds__(128) k_sep_combine(SepArgs A, SepAcc B) {
 }
 
 // ---- projection: radial contraction ----------------------------------------------
+constexpr int SEP_PRUN = 4;   // jobs of a run (k_sep_proj)
 struct SepPJob {
-  const double *rp;         // table of the class at this axial pair: [k][ld]
-  int ld, n, s0, nst;       // slots padded to 16, slots, first slot, slot tiles (1..4)
-  int nc;                   // terms
-  int t, kind, sa, sb, sec;
+  int64_t rp;               // offset of the class's table at this axial pair: [k][ld]
+  uint64_t fields;          // the terms' field components, seven bits each
+  int ld, n, s0, nst;       // slots padded to 16, slots, first slot, slot tiles (1..4; 0: an empty job)
+  int nc, sec;              // terms, sector
   int yoff, yld;            // Y of the class's first slot at this axial pair; stride between slots
 };
+static_assert(9 * 7 <= 64 && NFLD <= 128, "a job's nine field components fit 64 bits");
 
-// Y[p][(ri, z)] = sum_{c, r} R'_c[r][p] F_c(r, z) on v_mfma_f64_16x16x4: up to RT
-// tiles of 16 slots by CT tiles of 16 (ri, z) per wave, four radial points per
-// step.  The fields are read where k_fields put them.  As in k_sep_dens the
-// products of a step hide its loads; with few points RT = 1 gives four times
-// the waves.
+// One job with RT slot tiles (the loop as in sep_dens_job).
 template <int CT, int RT>
-__global__ void __launch_bounds__(64) k_sep_proj(SepArgs A, const SepPJob *__restrict__ jobs) {
-  const int w = A.act[blockIdx.y];
-  if (w == A.skip) return;
-  const SepPJob J = jobs[blockIdx.x];
+__device__ inline void sep_proj_job(const SepArgs &A, const SepPJob &J, int w, int y) {
   const int lane = threadIdx.x, mi = lane & 15, mk = lane >> 4;
   const int nz = A.nz, nr = A.nr, W = 2 * A.nzp, nr4 = (nr + 3) & ~3;
   const long G = (long)nz * nr;
@@ -578,54 +610,84 @@ __global__ void __launch_bounds__(64) k_sep_proj(SepArgs A, const SepPJob *__res
 #pragma unroll
     for (int c = 0; c < CT; ++c) C[q][c] = v4d{0, 0, 0, 0};
   const double *__restrict__ F = A.flds + (((size_t)w * 2 + J.sec) * 2 * NFLD) * G;
-  const double *__restrict__ R = J.rp + J.s0 + mi;
   // columns past the last axial point repeat it: finite, and multiplied by the
   // axial tables' zeros later
-  long col[CT];
+  int col[CT];
 #pragma unroll
   for (int c = 0; c < CT; ++c) {
-    const int k = min(((int)blockIdx.z * CT + c) * 16 + mi, W - 1);
-    col[c] = k < A.nzp ? min(k, nz - 1) : G + min(k - A.nzp, nz - 1);
+    const int k = min(((int)blockIdx.y * CT + c) * 16 + mi, W - 1);
+    col[c] = k < A.nzp ? min(k, nz - 1) : (int)G + min(k - A.nzp, nz - 1);
   }
-  auto load = [&](int c, int r0, double (&a)[RT], double (&b)[CT]) {
-    const int r = min(r0 + mk, nr - 1);          // table rows are zero past the last point
-    const double *f = F + 2 * (long)sep_field(J.kind, J.t, c, J.sa, J.sb) * G + (long)r * nz;
-#pragma unroll
-    for (int k = 0; k < CT; ++k) b[k] = f[col[k]];
-    const double *p = R + (size_t)(c * nr4 + r0 + mk) * J.ld;
-#pragma unroll
-    for (int q = 0; q < RT; ++q) a[q] = q < J.nst ? p[16 * q] : 0.0;
-  };
-  double an[RT], bn[CT];
-  int c = 0, r0 = 0;
-  load(0, 0, an, bn);
+  // step k: points r0 .. r0 + 3 of a term (table rows are zero past the last
+  // point, whose fields the lanes past it repeat)
+  const int rl = mk * nz, rt = (min(nr4 - 4 + mk, nr - 1) - (nr4 - 4)) * nz;
   const int nk = J.nc * (nr4 >> 2);
+  uint64_t fields = J.fields;
+  long fo = 2 * (long)(fields & 127) * G;
+  const double *__restrict__ p = A.tab + J.rp + J.s0 + mi + (size_t)mk * J.ld;
+  int r0 = 0;
+  double an[RT], bn[CT];
+  auto load = [&] {
+    const double *q = F + fo + (r0 + 4 < nr4 ? rl : rt);
+#pragma unroll
+    for (int k = 0; k < CT; ++k) bn[k] = q[col[k]];
+#pragma unroll
+    for (int k = 0; k < RT; ++k) an[k] = p[16 * k];
+  };
+  load();
   for (int k = 0; k < nk; ++k) {
     double a[RT], b[CT];
 #pragma unroll
     for (int q = 0; q < RT; ++q) a[q] = an[q];
 #pragma unroll
     for (int i = 0; i < CT; ++i) b[i] = bn[i];
-    r0 += 4;
-    if (r0 == nr4) { r0 = 0; ++c; }
-    if (k + 1 < nk) load(c, r0, an, bn);
+    // the next step, after the last one the last again
+    const bool more = k + 1 < nk, next = r0 + 4 == nr4;
+    fields = more && next ? fields >> 7 : fields;
+    fo = !more ? fo : (next ? 2 * (long)(fields & 127) * G : fo + 4 * nz);
+    r0 = !more ? r0 : (next ? 0 : r0 + 4);
+    p += more ? 4 * (size_t)J.ld : 0;
+    load();
+    loads_first();
 #pragma unroll
     for (int q = 0; q < RT; ++q)
-      if (q < J.nst)
 #pragma unroll
-        for (int i = 0; i < CT; ++i) C[q][i] = mfma64(a[q], b[i], C[q][i]);
+      for (int i = 0; i < CT; ++i) C[q][i] = mfma64(a[q], b[i], C[q][i]);
   }
-  double *out = A.zy + (size_t)blockIdx.y * A.ystride + J.yoff;
+  double *out = A.zy + (size_t)y * A.ystride + J.yoff;
 #pragma unroll
   for (int q = 0; q < RT; ++q)
-    if (q < J.nst)
 #pragma unroll
-      for (int i = 0; i < CT; ++i)
+    for (int i = 0; i < CT; ++i)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int k = ((int)blockIdx.z * CT + i) * 16 + mi, p = J.s0 + 16 * q + 4 * v + mk;
-          if (k < W && p < J.n) out[(size_t)p * J.yld + k] = C[q][i][v];
-        }
+      for (int v = 0; v < 4; ++v) {
+        const int k = ((int)blockIdx.y * CT + i) * 16 + mi, s = J.s0 + 16 * q + 4 * v + mk;
+        if (k < W && s < J.n) out[(size_t)s * J.yld + k] = C[q][i][v];
+      }
+}
+
+// Y[p][(ri, z)] = sum_{c, r} R'_c[r][p] F_c(r, z) on v_mfma_f64_16x16x4: up to RT
+// tiles of 16 slots by CT tiles of 16 (ri, z) per wave, four radial points per
+// step.  The fields are read where k_fields put them.  As in k_sep_dens the
+// products of a step hide its loads; with few points RT = 1 gives four times
+// the waves.
+template <int CT, int RT>
+__global__ void __launch_bounds__(64, RT > 1 ? 2 : 4) k_sep_proj(SepArgs A, const SepPJob *__restrict__ jobs, int njob) {
+  int y;
+  const SepPJob J = jobs[sep_job(njob, SEP_PRUN, A.na, y)];
+  const int w = A.act[y];
+  if (w == A.skip) return;
+  if (RT == 1) {
+    if (J.nst) sep_proj_job<CT, 1>(A, J, w, y);
+    return;
+  }
+  switch (J.nst) {
+    case 1: sep_proj_job<CT, 1>(A, J, w, y); break;
+    case 2: sep_proj_job<CT, 2>(A, J, w, y); break;
+    case 3: sep_proj_job<CT, 3>(A, J, w, y); break;
+    case 4: sep_proj_job<CT, 4>(A, J, w, y); break;
+    default: break;
+  }
 }
 
 // ---- projection: axial expansion ----------------------------------------------------
@@ -633,84 +695,112 @@ __global__ void __launch_bounds__(64) k_sep_proj(SepArgs A, const SepPJob *__res
 // the transpose of k_sep_z's product, [8 frequencies x (re, im)] x [(t, z)] by
 // [(t, z)] x elements, 16 elements per tile, up to SEP_EN tiles at a time.  A
 // lane holds two neighbouring axial points (16-byte loads, two matrix steps);
-// the five axial products of an element and z are formed in registers.  One
-// wave per slot and 8 frequencies.
-constexpr int SEP_EN = 3;
-__global__ void __launch_bounds__(256) k_sep_expand(SepArgs A, const SepSlot *__restrict__ slots,
-                                                    const int4 *__restrict__ elems, int nslot) {
-  const int id = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
-  if (id >= nslot) return;
-  const SepSlot S = slots[id];
+// the five axial products of an element and z are formed in registers, for MT
+// times 8 frequencies.
+constexpr int SEP_EN = 2;
+template <int MT, bool MEAN>
+__device__ inline void sep_expand_slot(const SepArgs &A, const SepSlot S, const int4 *__restrict__ elems) {
+  typedef double v2d __attribute__((ext_vector_type(2)));
+  constexpr int NT = MEAN ? 5 : 1, NX = MEAN ? 3 : 1;
   const int lane = threadIdx.x & 63, mi = lane & 15, mk = lane >> 4;
-  const bool mean = (S.mat & 1) == 0;
   const int nzp = A.nzp;
-  const int y = min((int)blockIdx.y * 8 + (mi >> 1), A.na - 1);
-  // a row of a point past the last repeats it: finite, not stored
-  const double *__restrict__ Y = A.zy + (size_t)y * A.ystride + S.zoff + (size_t)(mi & 1) * nzp + 2 * mk;
+  const double *Y[MT];
+  double *out[MT][4];      // where this lane stores (row 4 v + mk of the product), null: nowhere
+  const int out_slot = S.mat == 0 ? 0 : (S.mat == 1 ? 1 : (S.mat == 2 ? 3 : 2));
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    // a row of a point past the last repeats it: finite, not stored
+    const int y = min((int)(blockIdx.y * MT + m) * 8 + (mi >> 1), A.na - 1);
+    Y[m] = A.zy + (size_t)y * A.ystride + S.zoff + (size_t)(mi & 1) * nzp + 2 * mk;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int yo = (blockIdx.y * MT + m) * 8 + 2 * v + (mk >> 1), w = A.act[min(yo, A.na - 1)];
+      out[m][v] = yo < A.na && w != A.skip ? A.hsp + ((size_t)w * 8 + 2 * out_slot + (mk & 1)) * A.nxy : nullptr;
+    }
+  }
   const double *__restrict__ fz = A.fz + 2 * mk;
   const size_t xs = (size_t)A.dqp * nzp;
   const int4 *__restrict__ el = elems + S.first;
-  typedef double v2d __attribute__((ext_vector_type(2)));
-  const int out_slot = S.mat == 0 ? 0 : (S.mat == 1 ? 1 : (S.mat == 2 ? 3 : 2));
   for (int e0 = 0; e0 < S.count; e0 += 16 * SEP_EN) {
-    const int nt = min(SEP_EN, (S.count - e0 + 15) >> 4);
-    size_t oa[SEP_EN], ob[SEP_EN];
+    const double *fa[SEP_EN], *fb[SEP_EN];
     int off[SEP_EN];
 #pragma unroll
     for (int k = 0; k < SEP_EN; ++k) {
       const int4 r = el[min(e0 + 16 * k + mi, S.count - 1)];
-      off[k] = r.x; oa[k] = (size_t)r.y * nzp; ob[k] = (size_t)r.z * nzp;
+      off[k] = r.x; fa[k] = fz + (size_t)r.y * nzp; fb[k] = fz + (size_t)r.z * nzp;
     }
-    v4d C[SEP_EN];
+    const bool two = SEP_EN > 1 && e0 + 16 < S.count;     // the second tile has elements
+    v4d C[MT][SEP_EN];
 #pragma unroll
-    for (int k = 0; k < SEP_EN; ++k) C[k] = v4d{0, 0, 0, 0};
-    if (mean) {
-      for (int zb = 0; zb < nzp; zb += 8) {
-        v2d yv[5], a0[SEP_EN], a1[SEP_EN], a2[SEP_EN], b0[SEP_EN], b1[SEP_EN], b2[SEP_EN];
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int t = 0; t < 5; ++t) yv[t] = *(const v2d *)(Y + (size_t)(2 * t) * nzp + zb);
+      for (int k = 0; k < SEP_EN; ++k) C[m][k] = v4d{0, 0, 0, 0};
+    v2d yn[MT][NT], an[SEP_EN][NX], bn[SEP_EN][NX];
+    auto load = [&](int zb) {
 #pragma unroll
-        for (int k = 0; k < SEP_EN; ++k)
-          if (k < nt) {
-            a0[k] = *(const v2d *)(fz + oa[k] + zb); a1[k] = *(const v2d *)(fz + xs + oa[k] + zb);
-            a2[k] = *(const v2d *)(fz + 2 * xs + oa[k] + zb);
-            b0[k] = *(const v2d *)(fz + ob[k] + zb); b1[k] = *(const v2d *)(fz + xs + ob[k] + zb);
-            b2[k] = *(const v2d *)(fz + 2 * xs + ob[k] + zb);
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) yn[m][t] = *(const v2d *)(Y[m] + (size_t)(2 * t) * nzp + zb);
+#pragma unroll
+      for (int k = 0; k < SEP_EN; ++k)
+#pragma unroll
+        for (int x = 0; x < NX; ++x) {
+          an[k][x] = *(const v2d *)(fa[k] + x * xs + zb);
+          bn[k][x] = *(const v2d *)(fb[k] + x * xs + zb);
+        }
+    };
+    load(0);
+    for (int zb = 0; zb < nzp; zb += 8) {
+      v2d yv[MT][NT], X[SEP_EN][NT];
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) yv[m][t] = yn[m][t];
+#pragma unroll
+      for (int k = 0; k < SEP_EN; ++k)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          X[k][0][u] = an[k][0][u] * bn[k][0][u];
+          if constexpr (MEAN) {
+            X[k][1][u] = an[k][0][u] * bn[k][1][u];
+            X[k][2][u] = an[k][1][u] * bn[k][0][u];
+            X[k][3][u] = an[k][1][u] * bn[k][1][u];
+            X[k][4][u] = __builtin_fma(an[k][0][u], bn[k][2][u], an[k][2][u] * bn[k][0][u]);
           }
+        }
+      load(min(zb + 8, nzp - 8));
+      loads_first();
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int m = 0; m < MT; ++m) C[m][0] = mfma64(yv[m][t][u], X[0][t][u], C[m][0]);
+      if (two)
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+              C[m][SEP_EN - 1] = mfma64(yv[m][t][u], X[SEP_EN - 1][t][u], C[m][SEP_EN - 1]);
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        if (out[m][v])
+#pragma unroll
           for (int k = 0; k < SEP_EN; ++k)
-            if (k < nt) {
-              C[k] = mfma64(yv[0][u], a0[k][u] * b0[k][u], C[k]);
-              C[k] = mfma64(yv[1][u], a0[k][u] * b1[k][u], C[k]);
-              C[k] = mfma64(yv[2][u], a1[k][u] * b0[k][u], C[k]);
-              C[k] = mfma64(yv[3][u], a1[k][u] * b1[k][u], C[k]);
-              C[k] = mfma64(yv[4][u], __builtin_fma(a0[k][u], b2[k][u], a2[k][u] * b0[k][u]), C[k]);
-            }
-      }
-    } else {
-      for (int zb = 0; zb < nzp; zb += 8) {
-        const v2d yv = *(const v2d *)(Y + zb);
-#pragma unroll
-        for (int k = 0; k < SEP_EN; ++k)
-          if (k < nt) {
-            const v2d x = *(const v2d *)(fz + oa[k] + zb) * *(const v2d *)(fz + ob[k] + zb);
-#pragma unroll
-            for (int u = 0; u < 2; ++u) C[k] = mfma64(yv[u], x[u], C[k]);
-          }
-      }
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int yo = blockIdx.y * 8 + 2 * v + (mk >> 1);
-      if (yo >= A.na) continue;
-      const int w = A.act[yo];
-      if (w == A.skip) continue;
-      double *out = A.hsp + ((size_t)w * 8 + 2 * out_slot + (mk & 1)) * A.nxy;
-#pragma unroll
-      for (int k = 0; k < SEP_EN; ++k)
-        if (k < nt && e0 + 16 * k + mi < S.count) out[off[k]] = 2.0 * C[k][v];
-    }
+            if (e0 + 16 * k + mi < S.count) out[m][v][off[k]] = 2.0 * C[m][k][v];
   }
+}
+
+template <int MT>
+__global__ void __launch_bounds__(256) k_sep_expand(SepArgs A, const SepSlot *__restrict__ slots,
+                                                    const int4 *__restrict__ elems) {
+  const SepSlot S = slots[__builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)))];
+  if (S.count == 0) return;
+  if ((S.mat & 1) == 0) sep_expand_slot<MT, true>(A, S, elems);
+  else sep_expand_slot<MT, false>(A, S, elems);
 }
