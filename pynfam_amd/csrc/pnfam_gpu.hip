@@ -3634,10 +3634,12 @@ int stage_hamiltonian_sep(pnfam_gpu_ctx *h, int na, const int *act, const GridBu
 #undef SEP_P
       const SepSlot *sl = h->d_sep_slots[1].as<SepSlot>();
       const int4 *el = h->d_sep_elems[1].as<int4>();
-      if (nc > 8)
-        hipLaunchKernelGGL(k_sep_expand<2>, dim3(h->sep_nslot[1] / 4, (nc + 15) / 16), dim3(256), 0, h->stream, A, sl, el);
+      if (nc > 16)
+        hipLaunchKernelGGL(k_sep_expand_wide<4>, dim3(h->sep_nslot[1], (nc + 31) / 32), dim3(256), 0, h->stream, A, sl, el);
+      else if (nc > 8)
+        hipLaunchKernelGGL(k_sep_expand_wide<2>, dim3(h->sep_nslot[1], 1), dim3(128), 0, h->stream, A, sl, el);
       else
-        hipLaunchKernelGGL(k_sep_expand<1>, dim3(h->sep_nslot[1] / 4, 1), dim3(256), 0, h->stream, A, sl, el);
+        hipLaunchKernelGGL(k_sep_expand, dim3(h->sep_nslot[1] / 4), dim3(256), 0, h->stream, A, sl, el);
     }
   }
   HIP_TRY(hipGetLastError());

@@ -694,29 +694,25 @@ __global__ void __launch_bounds__(64, RT > 1 ? 2 : 4) k_sep_proj(SepArgs A, cons
 // h(a, b) = 2 sum_t sum_z Y_t[p](z) c_t1(z, a) c_t2(z, b) over the slot's elements:
 // the transpose of k_sep_z's product, [8 frequencies x (re, im)] x [(t, z)] by
 // [(t, z)] x elements, 16 elements per tile, up to SEP_EN tiles at a time.  A
-// lane holds two neighbouring axial points (16-byte loads, two matrix steps);
-// the five axial products of an element and z are formed in registers, for MT
-// times 8 frequencies.
+// lane holds two neighbouring axial points (16-byte loads, two matrix steps).
+// Up to 8 points: one wave per slot, the five axial products of an element and z
+// formed in registers.
 constexpr int SEP_EN = 2;
-template <int MT, bool MEAN>
+template <bool MEAN>
 __device__ inline void sep_expand_slot(const SepArgs &A, const SepSlot S, const int4 *__restrict__ elems) {
   typedef double v2d __attribute__((ext_vector_type(2)));
   constexpr int NT = MEAN ? 5 : 1, NX = MEAN ? 3 : 1;
   const int lane = threadIdx.x & 63, mi = lane & 15, mk = lane >> 4;
   const int nzp = A.nzp;
-  const double *Y[MT];
-  double *out[MT][4];      // where this lane stores (row 4 v + mk of the product), null: nowhere
+  // a row of a point past the last repeats it: finite, not stored
+  const double *__restrict__ Y =
+      A.zy + (size_t)min(mi >> 1, A.na - 1) * A.ystride + S.zoff + (size_t)(mi & 1) * nzp + 2 * mk;
+  double *out[4];          // where this lane stores (row 4 v + mk of the product), null: nowhere
   const int out_slot = S.mat == 0 ? 0 : (S.mat == 1 ? 1 : (S.mat == 2 ? 3 : 2));
 #pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    // a row of a point past the last repeats it: finite, not stored
-    const int y = min((int)(blockIdx.y * MT + m) * 8 + (mi >> 1), A.na - 1);
-    Y[m] = A.zy + (size_t)y * A.ystride + S.zoff + (size_t)(mi & 1) * nzp + 2 * mk;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int yo = (blockIdx.y * MT + m) * 8 + 2 * v + (mk >> 1), w = A.act[min(yo, A.na - 1)];
-      out[m][v] = yo < A.na && w != A.skip ? A.hsp + ((size_t)w * 8 + 2 * out_slot + (mk & 1)) * A.nxy : nullptr;
-    }
+  for (int v = 0; v < 4; ++v) {
+    const int yo = 2 * v + (mk >> 1), w = A.act[min(yo, A.na - 1)];
+    out[v] = yo < A.na && w != A.skip ? A.hsp + ((size_t)w * 8 + 2 * out_slot + (mk & 1)) * A.nxy : nullptr;
   }
   const double *__restrict__ fz = A.fz + 2 * mk;
   const size_t xs = (size_t)A.dqp * nzp;
@@ -730,17 +726,13 @@ __device__ inline void sep_expand_slot(const SepArgs &A, const SepSlot S, const 
       off[k] = r.x; fa[k] = fz + (size_t)r.y * nzp; fb[k] = fz + (size_t)r.z * nzp;
     }
     const bool two = SEP_EN > 1 && e0 + 16 < S.count;     // the second tile has elements
-    v4d C[MT][SEP_EN];
+    v4d C[SEP_EN];
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-      for (int k = 0; k < SEP_EN; ++k) C[m][k] = v4d{0, 0, 0, 0};
-    v2d yn[MT][NT], an[SEP_EN][NX], bn[SEP_EN][NX];
+    for (int k = 0; k < SEP_EN; ++k) C[k] = v4d{0, 0, 0, 0};
+    v2d yn[NT], an[SEP_EN][NX], bn[SEP_EN][NX];
     auto load = [&](int zb) {
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) yn[m][t] = *(const v2d *)(Y[m] + (size_t)(2 * t) * nzp + zb);
+      for (int t = 0; t < NT; ++t) yn[t] = *(const v2d *)(Y + (size_t)(2 * t) * nzp + zb);
 #pragma unroll
       for (int k = 0; k < SEP_EN; ++k)
 #pragma unroll
@@ -751,11 +743,9 @@ __device__ inline void sep_expand_slot(const SepArgs &A, const SepSlot S, const 
     };
     load(0);
     for (int zb = 0; zb < nzp; zb += 8) {
-      v2d yv[MT][NT], X[SEP_EN][NT];
+      v2d yv[NT], X[SEP_EN][NT];
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) yv[m][t] = yn[m][t];
+      for (int t = 0; t < NT; ++t) yv[t] = yn[t];
 #pragma unroll
       for (int k = 0; k < SEP_EN; ++k)
 #pragma unroll
@@ -773,34 +763,143 @@ __device__ inline void sep_expand_slot(const SepArgs &A, const SepSlot S, const 
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-          for (int m = 0; m < MT; ++m) C[m][0] = mfma64(yv[m][t][u], X[0][t][u], C[m][0]);
+        for (int t = 0; t < NT; ++t) C[0] = mfma64(yv[t][u], X[0][t][u], C[0]);
       if (two)
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
-          for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int m = 0; m < MT; ++m)
-              C[m][SEP_EN - 1] = mfma64(yv[m][t][u], X[SEP_EN - 1][t][u], C[m][SEP_EN - 1]);
+          for (int t = 0; t < NT; ++t) C[SEP_EN - 1] = mfma64(yv[t][u], X[SEP_EN - 1][t][u], C[SEP_EN - 1]);
     }
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int v = 0; v < 4; ++v)
+      if (out[v])
 #pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (out[m][v])
-#pragma unroll
-          for (int k = 0; k < SEP_EN; ++k)
-            if (e0 + 16 * k + mi < S.count) out[m][v][off[k]] = 2.0 * C[m][k][v];
+        for (int k = 0; k < SEP_EN; ++k)
+          if (e0 + 16 * k + mi < S.count) out[v][off[k]] = 2.0 * C[k][v];
   }
 }
 
-template <int MT>
 __global__ void __launch_bounds__(256) k_sep_expand(SepArgs A, const SepSlot *__restrict__ slots,
                                                     const int4 *__restrict__ elems) {
   const SepSlot S = slots[__builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)))];
   if (S.count == 0) return;
-  if ((S.mat & 1) == 0) sep_expand_slot<MT, true>(A, S, elems);
-  else sep_expand_slot<MT, false>(A, S, elems);
+  if ((S.mat & 1) == 0) sep_expand_slot<true>(A, S, elems);
+  else sep_expand_slot<false>(A, S, elems);
+}
+
+// The same for more than 8 points: the NW waves of a workgroup take the same slot for
+// 8 frequencies each, the axial products of up to SEP_EW element tiles and 8 axial
+// points formed once for all of them and kept in LDS in the layout of the
+// operand, the next chunk's loads in flight during the products of this one.
+// With a wave per slot for 16 frequencies, the products in registers, one wave
+// filled a SIMD's registers and the functions' loads were repeated for every 16
+// points: N_sh = 16, 128 points 2.25 ms, here 1.71 ms (0.40 ms at the peak matrix
+// rate; 2.1 GB read and as much written, 2.4 times what h holds: a slot's elements
+// lie in lines it shares with other slots).
+constexpr int SEP_EW = 4;
+template <int NW, bool MEAN>
+__device__ inline void sep_expand_wide(const SepArgs &A, const SepSlot S, const int4 *__restrict__ elems,
+                                       double (*__restrict__ buf)[5 * 2 * SEP_EW * 64]) {
+  typedef double v2d __attribute__((ext_vector_type(2)));
+  constexpr int NT = MEAN ? 5 : 1, NX = MEAN ? 3 : 1, NP = SEP_EW / NW;   // element and pair of z per thread
+  const int lane = threadIdx.x & 63, mi = lane & 15, mk = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), y0 = ((int)blockIdx.y * NW + wv) * 8;
+  const bool on = y0 < A.na;               // waves past the last point wait with the others
+  const int nzp = A.nzp;
+  // a row of a point past the last repeats it: finite, not stored
+  const double *__restrict__ Y =
+      A.zy + (size_t)min(y0 + (mi >> 1), A.na - 1) * A.ystride + S.zoff + (size_t)(mi & 1) * nzp + 2 * mk;
+  const int out_slot = S.mat == 0 ? 0 : (S.mat == 1 ? 1 : (S.mat == 2 ? 3 : 2));
+  const size_t xs = (size_t)A.dqp * nzp;
+  const int4 *__restrict__ el = elems + S.first;
+  const int q = threadIdx.x & 3;
+  for (int e0 = 0; e0 < S.count; e0 += 16 * SEP_EW) {
+    const int nk = min(SEP_EW, (S.count - e0 + 15) >> 4);
+    int fa[NP], fb[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int4 r = el[min(e0 + ((int)threadIdx.x >> 2) + 16 * NW * i, S.count - 1)];
+      fa[i] = r.y * nzp + 2 * q; fb[i] = r.z * nzp + 2 * q;
+    }
+    v4d C[SEP_EW];
+#pragma unroll
+    for (int k = 0; k < SEP_EW; ++k) C[k] = v4d{0, 0, 0, 0};
+    v2d yn[NT], an[NP][NX], bn[NP][NX];
+    auto load = [&](int zb) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i)
+#pragma unroll
+        for (int x = 0; x < NX; ++x) {
+          an[i][x] = *(const v2d *)(A.fz + x * xs + zb + fa[i]);
+          bn[i][x] = *(const v2d *)(A.fz + x * xs + zb + fb[i]);
+        }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) yn[t] = *(const v2d *)(Y + (size_t)(2 * t) * nzp + zb);
+    };
+    // value (t, u = z % 2, tile k, mk = z / 2, mi) at ((t 2 + u) SEP_EW + k) 64 + lane
+    auto form = [&](double *d) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        const int e = ((int)threadIdx.x >> 2) + 16 * NW * i;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          double *p = d + (u * SEP_EW + (e >> 4)) * 64 + q * 16 + (e & 15);
+          p[0] = an[i][0][u] * bn[i][0][u];
+          if constexpr (MEAN) {
+            p[1 * 2 * SEP_EW * 64] = an[i][0][u] * bn[i][1][u];
+            p[2 * 2 * SEP_EW * 64] = an[i][1][u] * bn[i][0][u];
+            p[3 * 2 * SEP_EW * 64] = an[i][1][u] * bn[i][1][u];
+            p[4 * 2 * SEP_EW * 64] = __builtin_fma(an[i][0][u], bn[i][2][u], an[i][2][u] * bn[i][0][u]);
+          }
+        }
+      }
+    };
+    load(0);
+    form(buf[0]);
+    __syncthreads();
+    int cur = 0;
+    for (int zb = 0; zb < nzp; zb += 8) {
+      v2d yv[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) yv[t] = yn[t];
+      load(min(zb + 8, nzp - 8));
+      loads_first();
+      const double *d = buf[cur] + lane;
+      if (on)
+#pragma unroll
+        for (int k = 0; k < SEP_EW; ++k)
+          if (k < nk)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+              for (int t = 0; t < NT; ++t) C[k] = mfma64(yv[t][u], d[((t * 2 + u) * SEP_EW + k) * 64], C[k]);
+      cur ^= 1;
+      if (zb + 8 < nzp) form(buf[cur]);
+      __syncthreads();
+    }
+    if (on) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int yo = y0 + 2 * v + (mk >> 1), w = A.act[min(yo, A.na - 1)];
+        if (yo < A.na && w != A.skip) {
+          double *out = A.hsp + ((size_t)w * 8 + 2 * out_slot + (mk & 1)) * A.nxy;
+#pragma unroll
+          for (int k = 0; k < SEP_EW; ++k)
+            if (e0 + 16 * k + mi < S.count) out[el[e0 + 16 * k + mi].x] = 2.0 * C[k][v];
+        }
+      }
+    }
+  }
+}
+
+// One slot per workgroup, in the order of k_sep_expand's workgroups of four.
+template <int NW>
+__global__ void __launch_bounds__(64 * NW, NW == 4 ? 3 : 2) k_sep_expand_wide(SepArgs A, const SepSlot *__restrict__ slots,
+                                                             const int4 *__restrict__ elems) {
+  __shared__ double buf[2][5 * 2 * SEP_EW * 64];
+  const int x = blockIdx.x & 7, i = blockIdx.x >> 3;
+  const SepSlot S = slots[((i >> 2) * 8 + x) * 4 + (i & 3)];
+  if (S.count == 0) return;
+  if ((S.mat & 1) == 0) sep_expand_wide<NW, true>(A, S, elems, buf);
+  else sep_expand_wide<NW, false>(A, S, elems, buf);
 }
