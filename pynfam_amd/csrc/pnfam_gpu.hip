@@ -2626,6 +2626,7 @@ struct pnfam_gpu_ctx {
   DevPtr d_sep_slots[2], d_sep_elems[2];         // density, projection
   int sep_nslot[2] = {0, 0}, sep_ndjob = 0, sep_nwork = 0, sep_npjob[2] = {0, 0}, sep_pjob0[2] = {0, 0};
   int sep_ct[2] = {1, 1}, sep_ncg[2] = {1, 1};   // density, projection: column tiles per wave, column groups
+  int sep_nct1 = 1;                              // column tiles of the projection
   SepAcc sep_acc{};
   long sep_zstride = 0, sep_ystride = 0, sep_arows = 0;
   double sep_flops_d = 0, sep_flops_p = 0;       // FLOP per point of the two halves; gen_: of the general kernels
@@ -3373,6 +3374,7 @@ int sep_build(pnfam_gpu_ctx *h) {
     const int nct = ((k ? W8 : W) + 15) / 16;
     h->sep_ncg[k] = (nct + 4) / 5;
     h->sep_ct[k] = (nct + h->sep_ncg[k] - 1) / h->sep_ncg[k];
+    if (k) h->sep_nct1 = nct;
   }
   std::vector<SepSlot> slots[2];
   std::vector<int4> elems[2];
@@ -3542,6 +3544,11 @@ bool sep_active(const pnfam_gpu_ctx *h) {
 // Points a pass of the separable stage takes at once, and the splits of its
 // density contraction: with few points the slots are split so that about 2 048
 // waves run.
+// Projection below eight points: one column tile per wave while that gives at most
+// this many waves (16 per CU; beyond, the operands read once per column tile cost
+// more than the shorter chains save: one point 21 us against 29 at N_sh = 8,
+// 18 against 25 at N_sh = 10).
+constexpr long SEP_PFEW = 4096;
 constexpr size_t SEP_CHUNK_BYTES = size_t(4) << 30;
 int sep_chunk(const pnfam_gpu_ctx *h, int na) {
   const size_t per = (size_t)std::max(h->sep_zstride, h->sep_ystride) * 8;
@@ -3615,16 +3622,16 @@ int stage_hamiltonian_sep(pnfam_gpu_ctx *h, int na, const int *act, const GridBu
     }
     { Prof pr(h, K_PROJECT, nc);
       const int v = nc >= 8 ? 1 : 0;   // four slot tiles per wave from eight points, one below
-      note(h, "k_sep_proj", h->sep_ct[1], v ? 4 : 1);
-      const dim3 grid(h->sep_npjob[v] * nc, h->sep_ncg[1]);
-      const int np = h->sep_npjob[v];
+      const int np = h->sep_npjob[v], ct = !v && (long)np * nc * h->sep_nct1 <= SEP_PFEW ? 1 : h->sep_ct[1];
+      note(h, "k_sep_proj", ct, v ? 4 : 1);
+      const dim3 grid(np * nc, (h->sep_nct1 + ct - 1) / ct);
       const SepPJob *pj = h->d_sep_pjobs.as<SepPJob>() + h->sep_pjob0[v];
 #define SEP_P(CT)                                                                                    \
   do {                                                                                               \
-    if (v) hipLaunchKernelGGL((k_sep_proj<CT, 4>), grid, dim3(64), 0, h->stream, A, pj, np);        \
-    else hipLaunchKernelGGL((k_sep_proj<CT, 1>), grid, dim3(64), 0, h->stream, A, pj, np);             \
+    if (v) hipLaunchKernelGGL((k_sep_proj<CT, 4>), grid, dim3(64), 0, h->stream, A, pj, np);         \
+    else hipLaunchKernelGGL((k_sep_proj<CT, 1>), grid, dim3(64), 0, h->stream, A, pj, np);           \
   } while (0)
-      switch (h->sep_ct[1]) {
+      switch (ct) {
         case 1: SEP_P(1); break;
         case 2: SEP_P(2); break;
         case 3: SEP_P(3); break;

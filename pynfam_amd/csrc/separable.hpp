@@ -598,8 +598,9 @@ struct SepPJob {
 };
 static_assert(9 * 7 <= 64 && NFLD <= 128, "a job's nine field components fit 64 bits");
 
-// One job with RT slot tiles (the loop as in sep_dens_job).
-template <int CT, int RT>
+// One job with RT slot tiles (the loop as in sep_dens_job); the loads of U steps
+// are in flight during the products of the U before.
+template <int CT, int RT, int U>
 __device__ inline void sep_proj_job(const SepArgs &A, const SepPJob &J, int w, int y) {
   const int lane = threadIdx.x, mi = lane & 15, mk = lane >> 4;
   const int nz = A.nz, nr = A.nr, W = 2 * A.nzp, nr4 = (nr + 3) & ~3;
@@ -609,7 +610,7 @@ __device__ inline void sep_proj_job(const SepArgs &A, const SepPJob &J, int w, i
   for (int q = 0; q < RT; ++q)
 #pragma unroll
     for (int c = 0; c < CT; ++c) C[q][c] = v4d{0, 0, 0, 0};
-  const double *__restrict__ F = A.flds + (((size_t)w * 2 + J.sec) * 2 * NFLD) * G;
+  const __amdgpu_buffer_rsrc_t F = rsrc64(A.flds + (((size_t)w * 2 + J.sec) * 2 * NFLD) * G, (int)(2 * NFLD * G));
   // columns past the last axial point repeat it: finite, and multiplied by the
   // axial tables' zeros later
   int col[CT];
@@ -623,36 +624,47 @@ __device__ inline void sep_proj_job(const SepArgs &A, const SepPJob &J, int w, i
   const int rl = mk * nz, rt = (min(nr4 - 4 + mk, nr - 1) - (nr4 - 4)) * nz;
   const int nk = J.nc * (nr4 >> 2);
   uint64_t fields = J.fields;
-  long fo = 2 * (long)(fields & 127) * G;
-  const double *__restrict__ p = A.tab + J.rp + J.s0 + mi + (size_t)mk * J.ld;
-  int r0 = 0;
-  double an[RT], bn[CT];
+  const int step = 4 * J.ld, G2 = 2 * (int)G;
+  const __amdgpu_buffer_rsrc_t R = rsrc64(A.tab + J.rp + J.s0, nk * step - J.s0);
+  const int ra = mk * J.ld + mi;
+  int r0 = 0, fo = (int)(fields & 127) * G2, p = 0;   // point, offsets in the fields and the table
+  double an[U][RT], bn[U][CT];
+  int kl = 0;               // the step the next load takes; after the last one the last again
   auto load = [&] {
-    const double *q = F + fo + (r0 + 4 < nr4 ? rl : rt);
 #pragma unroll
-    for (int k = 0; k < CT; ++k) bn[k] = q[col[k]];
+    for (int u = 0; u < U; ++u) {
+      const int q = r0 + 4 < nr4 ? rl : rt;
 #pragma unroll
-    for (int k = 0; k < RT; ++k) an[k] = p[16 * k];
+      for (int k = 0; k < CT; ++k) bn[u][k] = load64(F, col[k] + q, fo);
+#pragma unroll
+      for (int k = 0; k < RT; ++k) an[u][k] = load64(R, ra + 16 * k, p);
+      const bool more = ++kl < nk, next = r0 + 4 == nr4;
+      fields = more && next ? fields >> 7 : fields;
+      fo = !more ? fo : (next ? (int)(fields & 127) * G2 : fo + 4 * nz);
+      r0 = !more ? r0 : (next ? 0 : r0 + 4);
+      p += more ? step : 0;
+    }
   };
   load();
-  for (int k = 0; k < nk; ++k) {
-    double a[RT], b[CT];
+  for (int k = 0; k < nk; k += U) {
+    double a[U][RT], b[U][CT];
 #pragma unroll
-    for (int q = 0; q < RT; ++q) a[q] = an[q];
+    for (int u = 0; u < U; ++u) {
 #pragma unroll
-    for (int i = 0; i < CT; ++i) b[i] = bn[i];
-    // the next step, after the last one the last again
-    const bool more = k + 1 < nk, next = r0 + 4 == nr4;
-    fields = more && next ? fields >> 7 : fields;
-    fo = !more ? fo : (next ? 2 * (long)(fields & 127) * G : fo + 4 * nz);
-    r0 = !more ? r0 : (next ? 0 : r0 + 4);
-    p += more ? 4 * (size_t)J.ld : 0;
+      for (int q = 0; q < RT; ++q) a[u][q] = an[u][q];
+#pragma unroll
+      for (int i = 0; i < CT; ++i) b[u][i] = bn[u][i];
+    }
     load();
     loads_first();
 #pragma unroll
-    for (int q = 0; q < RT; ++q)
+    for (int u = 0; u < U; ++u) {
+      if (u > 0 && k + u >= nk) break;
 #pragma unroll
-      for (int i = 0; i < CT; ++i) C[q][i] = mfma64(a[q], b[i], C[q][i]);
+      for (int q = 0; q < RT; ++q)
+#pragma unroll
+        for (int i = 0; i < CT; ++i) C[q][i] = mfma64(a[u][q], b[u][i], C[q][i]);
+    }
   }
   double *out = A.zy + (size_t)y * A.ystride + J.yoff;
 #pragma unroll
@@ -668,24 +680,26 @@ __device__ inline void sep_proj_job(const SepArgs &A, const SepPJob &J, int w, i
 
 // Y[p][(ri, z)] = sum_{c, r} R'_c[r][p] F_c(r, z) on v_mfma_f64_16x16x4: up to RT
 // tiles of 16 slots by CT tiles of 16 (ri, z) per wave, four radial points per
-// step.  The fields are read where k_fields put them.  As in k_sep_dens the
-// products of a step hide its loads; with few points RT = 1 gives four times
-// the waves.
+// step.  The fields are read where k_fields put them.  With many points (RT = 4)
+// the products of a step hide its loads, as in k_sep_dens.  With few, a wave's
+// chain of steps (some 90) is what takes the time: one slot tile per wave, four
+// steps ahead, and where that leaves the device unfilled one column tile, eight
+// ahead (one point, N_sh = 8: 46 -> 21 us; N_sh = 16: 50 -> 39 us).
 template <int CT, int RT>
-__global__ void __launch_bounds__(64, RT > 1 ? 2 : 4) k_sep_proj(SepArgs A, const SepPJob *__restrict__ jobs, int njob) {
+__global__ void __launch_bounds__(64, RT > 1 ? 2 : 3) k_sep_proj(SepArgs A, const SepPJob *__restrict__ jobs, int njob) {
   int y;
   const SepPJob J = jobs[sep_job(njob, SEP_PRUN, A.na, y)];
   const int w = A.act[y];
   if (w == A.skip) return;
   if (RT == 1) {
-    if (J.nst) sep_proj_job<CT, 1>(A, J, w, y);
+    if (J.nst) sep_proj_job<CT, 1, CT == 1 ? 8 : 4>(A, J, w, y);
     return;
   }
   switch (J.nst) {
-    case 1: sep_proj_job<CT, 1>(A, J, w, y); break;
-    case 2: sep_proj_job<CT, 2>(A, J, w, y); break;
-    case 3: sep_proj_job<CT, 3>(A, J, w, y); break;
-    case 4: sep_proj_job<CT, 4>(A, J, w, y); break;
+    case 1: sep_proj_job<CT, 1, 1>(A, J, w, y); break;
+    case 2: sep_proj_job<CT, 2, 1>(A, J, w, y); break;
+    case 3: sep_proj_job<CT, 3, 1>(A, J, w, y); break;
+    case 4: sep_proj_job<CT, 4, 1>(A, J, w, y); break;
     default: break;
   }
 }
