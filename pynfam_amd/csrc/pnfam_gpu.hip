@@ -2101,11 +2101,6 @@ __device__ inline double wg_max(double v, double *red) {
   return s;
 }
 
-// vout <- vout - vin; partial max|vout|; for iter >= 2 also finalise the history
-// difference at slot ipos and its partial squared norm.
-// H: element type of the history (double; float on the mixed path, whose
-// pending raw vout stays FP64 in pdf, so the residual difference is formed
-// exactly, and whose dv is the step the last update wrote to dvin).
 // ifam's exit tests on the device, for the graph replay of the FP64 iteration
 // (pnfam_solver.f90:93-221): a point not yet done stops as converged (si below
 // the tolerance; its iteration count is the iteration index) or interrupted
@@ -2156,6 +2151,17 @@ __global__ void __launch_bounds__(1024) k_select(const double *__restrict__ si, 
   }
 }
 
+// vout <- vout - vin; partial max|vout|; for iter >= 2 also the partial squared
+// norm of the history difference at slot ipos, which an FP64 history forms again
+// in k_bro_dots (from values that kernel reads anyway), so that nothing but vout
+// is written here.
+// H: element type of the history (double; float on the mixed path, whose
+// pending raw vout stays FP64 in pdf, so the residual difference is formed
+// exactly, and whose dv is the step the last update wrote to dvin).
+// The Broyden kernels of an FP64 history run at the memory's rate (6 TB/s at 128
+// points): up to 8 pairs k, 4 + (k + 6) + (k + 5) vectors of 4 nxy pass per
+// iteration in resid, dots and update (7 + (k + 8) + (k + 5) with the difference
+// written here; N_sh = 16, 128 points, this kernel 617 -> 337 us).
 template <class H>
 __global__ void __launch_bounds__(BRO_WG) k_bro_resid(BroArgs B) {
   constexpr bool f64 = sizeof(H) == 8;
@@ -2181,8 +2187,10 @@ __global__ void __launch_bounds__(BRO_WG) k_bro_resid(BroArgs B) {
     vm = fmax(vm, fabs(vi[e]));
     if (hist) {
       const double f = d - (f64 ? (double)dfp[e] : qf[e]);
-      dfp[e] = (H)f;
-      dvp[e] = f64 ? (H)(vi[e] - (double)dvp[e]) : (H)qv[e];
+      if constexpr (!f64) {
+        dfp[e] = (H)f;
+        dvp[e] = (H)qv[e];
+      }
       nr += f * f;
     }
   }
@@ -2222,79 +2230,128 @@ __global__ void __launch_bounds__(64) k_bro_norm(BroArgs B) {
   B.scal[(size_t)w * 4 + 0] = (B.iter >= 2 && B.M > 0) ? (drop ? 0.0 : 1.0 / sqrt(s)) : 1.0;
 }
 
-// scale the history slot, then partial dots df_j . df_ipos and df_j . vout,
+// scale the history slot, then partial dots df_j . df_ipos and df_j . vout, up to
 // BRO_JB history vectors per pass over the new difference and vout.  An FP64
-// history keeps u_j = dv_j + alpha df_j in the dv slot from here on, the only
-// form the update reads (one vector per history entry instead of two)
+// history's slot holds the last vout and vin until here: its difference is formed,
+// scaled and stored in the first pass, u_j = dv_j + alpha df_j in the dv slot, the
+// only form the update reads (one vector per history entry instead of two)
 constexpr int BRO_JB = 8;
+template <class H, int NJ, bool FIRST>
+__device__ inline void bro_dots_pass(const BroArgs &B, int w, int j0, double normi, double *red) {
+  constexpr bool f64 = sizeof(H) == 8;
+  const long N = B.N;
+  H *dfp = (H *)B.df + ((size_t)w * B.M + B.ipos) * N;
+  H *dvp = (H *)B.dv + ((size_t)w * B.M + B.ipos) * N;
+  const double *vo = B.vout + (size_t)w * N, *vi = B.vin + (size_t)w * N;
+  double g[NJ], v[NJ];
+  const H *hj[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    g[j] = 0.0; v[j] = 0.0;
+    hj[j] = (const H *)B.df + ((size_t)w * B.M + j0 + j) * N;
+  }
+  const int own = B.ipos - j0;              // the new difference itself (what memory held before it does not count)
+  for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < N; e += (long)gridDim.x * blockDim.x) {
+    const double o = vo[e];
+    double a[NJ], p;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) a[j] = hj[j][e];
+    if constexpr (f64 && FIRST) {
+      const double f = o - dfp[e], q = vi[e] - dvp[e];
+      p = f * normi;
+      dfp[e] = p;
+      dvp[e] = __builtin_fma(B.alpha, p, q * normi);
+    } else if constexpr (FIRST) {
+      const H f = (H)(dfp[e] * normi);
+      dfp[e] = f;
+      dvp[e] = (H)(dvp[e] * normi);
+      p = f;
+    } else {
+      p = dfp[e];
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const double x = j == own ? p : a[j];
+      g[j] += x * p;
+      v[j] += x * o;
+    }
+  }
+  // the 2 NJ sums of the pass together: per value the shuffle tree and wave order
+  // of wg_sum, one LDS exchange for all of them
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+    for (int o = 32; o > 0; o >>= 1) {
+      g[j] += __shfl_down(g[j], o, 64);
+      v[j] += __shfl_down(v[j], o, 64);
+    }
+  const int lane = threadIdx.x % 64, wid = threadIdx.x / 64;
+  __syncthreads();
+  if (lane == 0)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) { red[(2 * j) * (BRO_WG / 64) + wid] = g[j]; red[(2 * j + 1) * (BRO_WG / 64) + wid] = v[j]; }
+  __syncthreads();
+  if (threadIdx.x < 2 * NJ) {
+    double t = 0.0;
+    for (int q = 0; q < BRO_WG / 64; ++q) t += red[threadIdx.x * (BRO_WG / 64) + q];
+    *bro_part(B, w, 2 + 2 * j0 + threadIdx.x, blockIdx.x) = t;
+  }
+}
+
+template <class H, bool FIRST>
+__device__ inline void bro_dots_step(const BroArgs &B, int w, int j0, double normi, double *red) {
+  switch (min(BRO_JB, B.iter_used - j0)) {
+    case 1: bro_dots_pass<H, 1, FIRST>(B, w, j0, normi, red); break;
+    case 2: bro_dots_pass<H, 2, FIRST>(B, w, j0, normi, red); break;
+    case 3: bro_dots_pass<H, 3, FIRST>(B, w, j0, normi, red); break;
+    case 4: bro_dots_pass<H, 4, FIRST>(B, w, j0, normi, red); break;
+    case 5: bro_dots_pass<H, 5, FIRST>(B, w, j0, normi, red); break;
+    case 6: bro_dots_pass<H, 6, FIRST>(B, w, j0, normi, red); break;
+    case 7: bro_dots_pass<H, 7, FIRST>(B, w, j0, normi, red); break;
+    default: bro_dots_pass<H, 8, FIRST>(B, w, j0, normi, red); break;
+  }
+}
+
 template <class H>
 __global__ void __launch_bounds__(BRO_WG) k_bro_dots(BroArgs B) {
   __shared__ double red[2 * BRO_JB * (BRO_WG / 64)];
   const int w = B.act[blockIdx.y];
   if (w == B.skip) return;
   bro_iter(B, w);
-  const long N = B.N;
+  if (B.iter_used < 1) return;
   const double normi = B.scal[(size_t)w * 4 + 0];
-  H *dfp = (H *)B.df + ((size_t)w * B.M + B.ipos) * N;
-  H *dvp = (H *)B.dv + ((size_t)w * B.M + B.ipos) * N;
-  const double *vo = B.vout + (size_t)w * N;
-  const long e0 = (long)blockIdx.x * blockDim.x + threadIdx.x, es = (long)gridDim.x * blockDim.x;
-  if (B.iter >= 2)
-    for (long e = e0; e < N; e += es) {
-      if constexpr (sizeof(H) == 8) {
-        const double f = dfp[e] * normi, v = dvp[e] * normi;
-        dfp[e] = f;
-        dvp[e] = __builtin_fma(B.alpha, f, v);
-      } else {
-        dfp[e] = (H)(dfp[e] * normi); dvp[e] = (H)(dvp[e] * normi);
-      }
-    }
+  bro_dots_step<H, true>(B, w, 0, normi, red);
+  for (int j0 = BRO_JB; j0 < B.iter_used; j0 += BRO_JB) bro_dots_step<H, false>(B, w, j0, normi, red);
+}
 
-  for (int j0 = 0; j0 < B.iter_used; j0 += BRO_JB) {
-    const int nj = min(BRO_JB, B.iter_used - j0);
-    double g[BRO_JB], v[BRO_JB];
-#pragma unroll
-    for (int j = 0; j < BRO_JB; ++j) { g[j] = 0.0; v[j] = 0.0; }
-    const H *df0 = (const H *)B.df + ((size_t)w * B.M + j0) * N;
-    for (long e = e0; e < N; e += es) {
-      const double p = dfp[e], o = vo[e];
-#pragma unroll
-      for (int j = 0; j < BRO_JB; ++j) {
-        if (j < nj) {
-          const double a = df0[(size_t)j * N + e];
-          g[j] += a * p;
-          v[j] += a * o;
-        }
-      }
-    }
-    // the 2 BRO_JB sums of the chunk together: per value the shuffle tree and
-    // wave order of wg_sum, one LDS exchange for all of them
-#pragma unroll
-    for (int j = 0; j < BRO_JB; ++j)
-      for (int o = 32; o > 0; o >>= 1) {
-        g[j] += __shfl_down(g[j], o, 64);
-        v[j] += __shfl_down(v[j], o, 64);
-      }
-    const int lane = threadIdx.x % 64, wid = threadIdx.x / 64;
-    __syncthreads();
-    if (lane == 0)
-#pragma unroll
-      for (int j = 0; j < BRO_JB; ++j) { red[(2 * j) * (BRO_WG / 64) + wid] = g[j]; red[(2 * j + 1) * (BRO_WG / 64) + wid] = v[j]; }
-    __syncthreads();
-    if (threadIdx.x < 2 * nj) {
-      double t = 0.0;
-      for (int q = 0; q < BRO_WG / 64; ++q) t += red[threadIdx.x * (BRO_WG / 64) + q];
-      *bro_part(B, w, 2 + 2 * j0 + threadIdx.x, blockIdx.x) = t;
-    }
-  }
+// Lane l's value, l uniform.
+__device__ inline double wave_read(double v, int l) {
+  const long b = __builtin_bit_cast(long, v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)b, l), hi = __builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
+  return __builtin_bit_cast(double, (long)(((unsigned long)hi << 32) | lo));
+}
+
+// Largest value of the wave (every lane must hold a number).
+__device__ inline double wave_max(double v) {
+  auto step = [&](auto f) {
+    const long b = __builtin_bit_cast(long, v);
+    const unsigned lo = f((int)(unsigned)b), hi = f((int)(unsigned)(b >> 32));
+    v = fmax(v, __builtin_bit_cast(double, (long)(((unsigned long)hi << 32) | lo)));
+  };
+  // lanes without a partner keep their own value; lane 63 ends with the whole wave's
+  step([](int x) { return __builtin_amdgcn_update_dpp(x, x, 0x111, 0xf, 0xf, false); });   // row_shr:1
+  step([](int x) { return __builtin_amdgcn_update_dpp(x, x, 0x112, 0xf, 0xf, false); });
+  step([](int x) { return __builtin_amdgcn_update_dpp(x, x, 0x114, 0xf, 0xf, false); });
+  step([](int x) { return __builtin_amdgcn_update_dpp(x, x, 0x118, 0xf, 0xf, false); });
+  step([](int x) { return __builtin_amdgcn_update_dpp(x, x, 0x142, 0xa, 0xf, false); });   // row_bcast:15
+  step([](int x) { return __builtin_amdgcn_update_dpp(x, x, 0x143, 0xc, 0xf, false); });   // row_bcast:31
+  return wave_read(v, 63);
 }
 
 // Gram row update, beta = (w0^2+1) I + offdiag(Gram), gamma = beta^-1 work
 // (Gauss-Jordan on one workgroup per frequency)
-__global__ void __launch_bounds__(256) k_bro_solve(BroArgs B) {
+__global__ void __launch_bounds__(512) k_bro_solve(BroArgs B) {
   __shared__ double a[BRO_MAXM][2 * BRO_MAXM + 1];
   __shared__ double work[BRO_MAXM];
-  __shared__ double fac[BRO_MAXM];
   const int w = B.act[blockIdx.x];
   if (w == B.skip) return;
   bro_iter(B, w);
@@ -2323,7 +2380,7 @@ __global__ void __launch_bounds__(256) k_bro_solve(BroArgs B) {
   __syncthreads();
   const double w0 = 0.010;
   // rows over the waves, columns over the lanes (no integer division per element)
-  const int gl = threadIdx.x & 63, gw = threadIdx.x >> 6, gnw = blockDim.x >> 6;
+  const int gl = threadIdx.x & 63, gw = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), gnw = blockDim.x >> 6;
   for (int i = gw; i < k; i += gnw)
     for (int j = gl; j < 2 * k; j += 64) {
       double v;
@@ -2332,53 +2389,44 @@ __global__ void __launch_bounds__(256) k_bro_solve(BroArgs B) {
       a[i][j] = v;
     }
   __syncthreads();
-  // Gauss-Jordan with partial pivoting (the first largest |a[i][c]|), three
-  // barriers per column: wave 0 finds the pivot; the rows are swapped, row c
-  // scaled and the elimination factors taken in one pass; then the elimination.
-  __shared__ int piv_s;
-  __shared__ double pval_s;
+  // Gauss-Jordan with partial pivoting (the first largest |a[i][c]|).  What a
+  // column takes is latency, so it has one barrier (three, and the shuffles of the
+  // search through LDS: 65 us for 30 pairs, now 40): rows stay where they are
+  // (lane l of every wave holds the row at position l and swaps it there), every
+  // wave finds the pivot by itself, column c and the pivot row are only read in
+  // step c (columns up to c are not needed any more), and the pivot row is scaled
+  // when the next step reads it.
+  int row = gl;
+  double dl = 1.0;                          // scale of the last pivot row (position c - 1)
   for (int c = 0; c < k; ++c) {
-    if (threadIdx.x < 64) {
-      int bi = c;
-      double bv = -1.0;
-      for (int i = c + threadIdx.x; i < k; i += 64) {
-        const double x = fabs(a[i][c]);
-        if (x > bv) { bv = x; bi = i; }
-      }
-      for (int o = 32; o > 0; o >>= 1) {
-        const double ov = __shfl_xor(bv, o, 64);
-        const int oi = __shfl_xor(bi, o, 64);
-        if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-      }
-      if (threadIdx.x == 0) { piv_s = bi; pval_s = a[bi][c]; }
-    }
-    __syncthreads();
-    // rows c and piv are written only by the column loop, which also records
-    // the factor of row piv (the old a[c][c]) from its own read
-    const int piv = piv_s;
-    const double d = 1.0 / pval_s;
-    for (int i = threadIdx.x; i < k; i += blockDim.x)
-      if (i != piv && i != c) fac[i] = a[i][c];
-    for (int j = threadIdx.x; j < 2 * k; j += blockDim.x) {
-      const double t = a[c][j], pv = a[piv][j];
-      if (piv != c) {
-        if (j == c) fac[piv] = t;
-        a[piv][j] = t;
-      }
-      a[c][j] = pv * d;
-    }
-    __syncthreads();
+    const bool cand = gl >= c && gl < k;
+    const double av = cand ? a[row][c] : 0.0;
+    const double x = cand && fabs(av) > -1.0 ? fabs(av) : -1.0;
+    const double big = wave_max(x);
+    const int pos = __builtin_ctzll(__ballot(cand && x == big));
+    const double d = 1.0 / wave_read(av, pos);
+    const int rp = __builtin_amdgcn_readlane(row, pos), rc = __builtin_amdgcn_readlane(row, c);
+    row = gl == c ? rp : (gl == pos ? rc : row);
     for (int i = gw; i < k; i += gnw) {
       if (i == c) continue;
-      const double f = fac[i];
-      for (int j = gl; j < 2 * k; j += 64) a[i][j] -= f * a[c][j];
+      const int r = __builtin_amdgcn_readlane(row, i);
+      const double sc = i == c - 1 ? dl : 1.0, f = a[r][c] * sc;
+      for (int j = gl; j < 2 * k; j += 64)
+        if (j > c) a[r][j] = __builtin_fma(-f, a[rp][j] * d, a[r][j] * sc);
     }
+    dl = d;
     __syncthreads();
   }
-  for (int i = threadIdx.x; i < k; i += blockDim.x) {
+  // position k - 1 still waits for its scale
+  for (int i0 = 0; i0 < k; i0 += blockDim.x) {
+    const int i = i0 + (int)threadIdx.x;
     double g = 0.0;
-    for (int j = 0; j < k; ++j) g += a[j][k + i] * work[j];   // beta(j,i)
-    B.coef[(size_t)w * M + i] = g;
+    for (int j = 0; j < k; ++j) {           // beta(j,i)
+      const double b = a[__builtin_amdgcn_readlane(row, j)][k + min(i, k - 1)];
+      g = __builtin_fma(j == k - 1 ? b * dl : b, work[j], g);
+    }
+    if (i < k)
+      B.coef[(size_t)w * M + i] = g;
   }
 }
 
@@ -4921,7 +4969,7 @@ static int bro_run(pnfam_gpu_ctx *h, int M, int iter, double alpha, int na, cons
     { Prof pr(h, K_BRO_DOTS, na);
       if (hist32) hipLaunchKernelGGL(k_bro_dots<float>, dim3(nwg_it, na), dim3(BRO_WG), 0, st, B);
       else hipLaunchKernelGGL(k_bro_dots<double>, dim3(nwg_it, na), dim3(BRO_WG), 0, st, B); }
-    { Prof pr(h, K_BRO_SOLVE, na); hipLaunchKernelGGL(k_bro_solve, dim3(na), dim3(256), 0, st, B); }
+    { Prof pr(h, K_BRO_SOLVE, na); hipLaunchKernelGGL(k_bro_solve, dim3(na), dim3(512), 0, st, B); }
   }
   { Prof pr(h, K_BRO_UPDATE, na);
     if (hist32) hipLaunchKernelGGL(k_bro_update<float>, dim3(nwg_it, na), dim3(BRO_WG), 0, st, B, mode);
