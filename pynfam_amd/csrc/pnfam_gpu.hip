@@ -2497,17 +2497,40 @@ __global__ void __launch_bounds__(256) k_contract(const double *__restrict__ vin
   if (threadIdx.x == 0) { part[o] = a; part[o + 1] = b; }
 }
 
+// res: where the host reads the iteration's results (mapped memory: si, max|vin| and
+// S of every point), null: nowhere.
+struct HostRes {
+  double *res;
+  const double *si, *vmax;
+  int npts;
+};
 __global__ void k_contract_fin(const double *__restrict__ part, int nwg, double *__restrict__ S,
-                               const int *__restrict__ act, int nop, int skip) {
+                               const int *__restrict__ act, int nop, int skip, HostRes R) {
   const int w = act[blockIdx.x];
   if (w == skip) return;
-  const int z = threadIdx.x;
-  if (z >= nop) return;
-  const double *p = part + ((size_t)w * nop + z) * nwg * 2;
+  // one operator z per workgroup (one wave); the partials come in together and are
+  // added in order
+  __shared__ double p[128];
+  const int z = blockIdx.y;
+  const double *q = part + ((size_t)w * nop + z) * nwg * 2;
   double a = 0.0, b = 0.0;
-  for (int k = 0; k < nwg; ++k) { a += p[2 * k]; b += p[2 * k + 1]; }
+  for (int k0 = 0; k0 < nwg; k0 += 64) {
+    const int n = min(64, nwg - k0);
+    __syncthreads();
+    for (int e = threadIdx.x; e < 2 * n; e += 64) p[e] = q[2 * k0 + e];
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int k = 0; k < n; ++k) { a += p[2 * k]; b += p[2 * k + 1]; }
+  }
+  if (threadIdx.x > 0) return;
   S[((size_t)w * nop + z) * 2] = -a / PI;
   S[((size_t)w * nop + z) * 2 + 1] = -b / PI;
+  if (R.res && z == 0) {
+    R.res[w] = R.si[w];
+    R.res[R.npts + w] = R.vmax[w];
+    R.res[2 * R.npts + 2 * w] = -a / PI;
+    R.res[2 * R.npts + 2 * w + 1] = -b / PI;
+  }
 }
 
 // dst = src for every active point's [w][n] slot
@@ -4979,7 +5002,7 @@ static int bro_run(pnfam_gpu_ctx *h, int M, int iter, double alpha, int na, cons
 }
 
 // Strength (and cross-terms) of the active points from their current amplitudes.
-static int contract_active(pnfam_gpu_ctx *h, int na, const int *dact) {
+static int contract_active(pnfam_gpu_ctx *h, int na, const int *dact, HostRes R = {}) {
   hipStream_t st = h->stream;
   const int cnwg = 64;
   { Prof pr(h, K_CONTRACT, na);
@@ -4991,10 +5014,10 @@ static int contract_active(pnfam_gpu_ctx *h, int na, const int *dact) {
                          h->nxy, h->nx, h->skip_slot); }
   { Prof pr(h, K_CONTRACT_FIN, na);
     hipLaunchKernelGGL(k_contract_fin, dim3(na), dim3(64), 0, st, h->d_cpart.as<double>(), cnwg, h->d_S.as<double>(),
-                       dact, 1, h->skip_slot);
+                       dact, 1, h->skip_slot, R);
     if (h->nx > 0)
-      hipLaunchKernelGGL(k_contract_fin, dim3(na), dim3(64), 0, st, h->d_xpart.as<double>(), cnwg,
-                         h->d_xs.as<double>(), dact, h->nx, h->skip_slot); }
+      hipLaunchKernelGGL(k_contract_fin, dim3(na, h->nx), dim3(64), 0, st, h->d_xpart.as<double>(), cnwg,
+                         h->d_xs.as<double>(), dact, h->nx, h->skip_slot, HostRes{}); }
   HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -5145,7 +5168,7 @@ static int solve_core(pnfam_gpu_ctx *h, int32_t npts, const double *re_w, const 
   }
   const double *e1 = h->bminus ? h->d_Ep.as<double>() : h->d_En.as<double>();
   const double *e2 = h->bminus ? h->d_En.as<double>() : h->d_Ep.as<double>();
-  std::vector<int> act, act64, actlo;
+  std::vector<int> act, act64, actlo, sent;   // sent: the list d_act holds
   const double tau = h->mix_tau;
   const long nq = 4 * nxy;   // doubles of H20/H02 (re, im) per frequency
   // PNFAM_GPU_TRACE=1: one line per iteration on stderr (active points, BF16
@@ -5358,16 +5381,24 @@ static int solve_core(pnfam_gpu_ctx *h, int32_t npts, const double *re_w, const 
     }
     const int na = (int)act.size();
     int *dact = h->d_act.as<int>();
-    std::memcpy(h->pin_act, act.data(), na * 4);
-    HIP_TRY(hipMemcpyAsync(dact, h->pin_act, na * 4, hipMemcpyHostToDevice, st));
+    // the device keeps the list until points retire; the results come back through
+    // mapped memory (k_contract_fin): a copy is some 10 us of an iteration of 130 to
+    // 180 (one point, N_sh = 8)
+    if (act != sent) {
+      std::memcpy(h->pin_act, act.data(), na * 4);
+      HIP_TRY(hipMemcpyAsync(dact, h->pin_act, na * 4, hipMemcpyHostToDevice, st));
+      sent = act;
+    }
     // vin = 0 at iteration 0 of a fresh start, so H(vin) = 0 exactly there and
     // the chain is not run
     const bool use_h = !skip_res && iter >= first_h;
     if (use_h && !act64.empty()) {
       const int n64 = (int)act64.size();
-      int *d64 = h->d_act64.as<int>();
-      std::memcpy(h->pin_act + npts, act64.data(), n64 * 4);
-      HIP_TRY(hipMemcpyAsync(d64, h->pin_act + npts, n64 * 4, hipMemcpyHostToDevice, st));
+      int *d64 = n64 == na ? dact : h->d_act64.as<int>();   // all active points: the same list
+      if (n64 < na) {
+        std::memcpy(h->pin_act + npts, act64.data(), n64 * 4);
+        HIP_TRY(hipMemcpyAsync(d64, h->pin_act + npts, n64 * 4, hipMemcpyHostToDevice, st));
+      }
       if (int e = stage_qp2sp(h, h->d_vin.as<double>(), n64, d64)) return e;
       if (int e = stage_hamiltonian(h, n64, d64)) return e;
       if (int e = stage_sp2qp(h, n64, d64)) return e;
@@ -5428,11 +5459,9 @@ static int solve_core(pnfam_gpu_ctx *h, int32_t npts, const double *re_w, const 
       dlag = h->d_lag.as<int>();
     }
     if (int e = bro_run(h, M, iter, o->alpha_mix, na, dact, hist32, ddrop, mixed, nullptr, dlag)) return e;
-    if (int e = contract_active(h, na, dact)) return e;
-    double *pr = h->pin_res;
-    HIP_TRY(hipMemcpyAsync(pr, h->d_si.p, npts * 8, hipMemcpyDeviceToHost, st));
-    if (mixed) HIP_TRY(hipMemcpyAsync(pr + npts, h->d_vmax.p, npts * 8, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(pr + 2 * npts, h->d_S.p, 2 * npts * 8, hipMemcpyDeviceToHost, st));
+    const double *pr = h->pin_res;
+    if (int e = contract_active(h, na, dact, HostRes{h->pin_res, h->d_si.as<double>(), h->d_vmax.as<double>(), npts}))
+      return e;
     HIP_TRY(hipStreamSynchronize(st));
     for (int w : act) {
       b.si[w] = pr[w];
