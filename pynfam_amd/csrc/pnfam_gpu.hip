@@ -3662,14 +3662,24 @@ int stage_hamiltonian_sep(pnfam_gpu_ctx *h, int na, const int *act, const GridBu
       const int ns = sep_split(h, nc, gb.split);
       note(h, "k_sep_dens", h->sep_ct[0], ns);
       const int zt = (h->sep_nz + 15) / 16, zg = (zt + 2) / 3;
-      const dim3 zgrid(h->sep_nslot[0] / 4, (nc + 7) / 8, zg);
       const SepSlot *sl = h->d_sep_slots[0].as<SepSlot>();
       const int4 *el = h->d_sep_elems[0].as<int4>();
+#define SEP_Z(ZT)                                                                                                      \
+  do {                                                                                                                 \
+    if (nc > 16)                                                                                                       \
+      hipLaunchKernelGGL((k_sep_z_wide<ZT, 4>), dim3(h->sep_nslot[0], (nc + 31) / 32, zg), dim3(256), 0, h->stream, A, \
+                         sl, el);                                                                                      \
+    else if (nc > 8)                                                                                                   \
+      hipLaunchKernelGGL((k_sep_z_wide<ZT, 2>), dim3(h->sep_nslot[0], 1, zg), dim3(128), 0, h->stream, A, sl, el);     \
+    else                                                                                                               \
+      hipLaunchKernelGGL(k_sep_z<ZT>, dim3(h->sep_nslot[0] / 4, 1, zg), dim3(256), 0, h->stream, A, sl, el);           \
+  } while (0)
       switch ((zt + zg - 1) / zg) {
-        case 1: hipLaunchKernelGGL(k_sep_z<1>, zgrid, dim3(256), 0, h->stream, A, sl, el); break;
-        case 2: hipLaunchKernelGGL(k_sep_z<2>, zgrid, dim3(256), 0, h->stream, A, sl, el); break;
-        default: hipLaunchKernelGGL(k_sep_z<3>, zgrid, dim3(256), 0, h->stream, A, sl, el); break;
+        case 1: SEP_Z(1); break;
+        case 2: SEP_Z(2); break;
+        default: SEP_Z(3); break;
       }
+#undef SEP_Z
       const dim3 grid(h->sep_ndjob * nc, h->sep_ncg[0] * ns);
 #define SEP_D(CT) hipLaunchKernelGGL(k_sep_dens<CT>, grid, dim3(64), 0, h->stream, A, h->d_sep_djobs.as<SepDJob>(), h->sep_ndjob, h->sep_ncg[0], ns)
       switch (h->sep_ct[0]) {

@@ -417,6 +417,130 @@ __global__ void __launch_bounds__(256) k_sep_z(SepArgs A, const SepSlot *__restr
   else sep_z_slot<ZT, false>(A, S, elems);
 }
 
+// The same for more than 8 points: the NW waves of a workgroup take the same slot for
+// 8 frequencies each, the axial products of 8 elements formed once for all of them
+// and kept in LDS in the layout of the operand, the loads of the next 8 in flight
+// during the products of these.  In k_sep_z every wave loads the functions for
+// itself, and the L1 serves those at its limit: N_sh = 16, 128 points 1.75 ms,
+// here 1.31 ms (0.34 ms at the peak matrix rate, and 1.9 GB of Z to write).
+template <int ZT, int NW, bool MEAN>
+__device__ inline void sep_z_wide(const SepArgs &A, const SepSlot S, const int4 *__restrict__ elems,
+                                  double (*__restrict__ buf)[2 * 4 * ZT * 64]) {
+  typedef double v2d __attribute__((ext_vector_type(2)));
+  constexpr int NX = MEAN ? 4 : 1, NP = (ZT + NW - 1) / NW;   // products' element and pair of z per thread
+  const int tid = threadIdx.x, lane = tid & 63, mi = lane & 15, mk = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), y0 = ((int)blockIdx.y * NW + wv) * 8;
+  const bool on = y0 < A.na;               // waves past the last point wait with the others
+  const double *__restrict__ rho =
+      A.rsp + ((size_t)A.act[min(y0 + (mi >> 1), A.na - 1)] * 8 + 2 * A.slot_of[S.mat] + (mi & 1)) * A.nxy;
+  const size_t xs = (size_t)A.dqp * A.nzp;
+  const int4 *__restrict__ el = elems + S.first;
+  const int n = S.count;
+  // this thread's products: element pe[i] of the chunk, axial points zp[i] and + 1
+  int pe[NP], zp[NP], at[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int q = min(tid + 64 * NW * i, 64 * ZT - 1), z = 2 * (q % (8 * ZT));
+    pe[i] = q / (8 * ZT);
+    zp[i] = min((int)blockIdx.z * ZT * 16 + z, A.nzp - 2);
+    at[i] = ((pe[i] >> 2) * NX * ZT + (z >> 4)) * 64 + (pe[i] & 3) * 16 + (z & 15);
+  }
+  v4d C[ZT][NX];
+#pragma unroll
+  for (int t = 0; t < ZT; ++t)
+#pragma unroll
+    for (int k = 0; k < NX; ++k) C[t][k] = v4d{0, 0, 0, 0};
+  v2d f[NP][4];
+  int4 rx[NP];
+  int rr[2];
+  double vn[2];
+  auto next = [&](int e0) {                // list entries of a chunk
+#pragma unroll
+    for (int i = 0; i < NP; ++i) rx[i] = el[min(e0 + pe[i], n - 1)];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) rr[s] = el[min(e0 + 4 * s + mk, n - 1)].x;
+  };
+  auto load = [&] {                        // its functions and matrix elements
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const double *fa = A.fz + (size_t)rx[i].y * A.nzp + zp[i], *fb = A.fz + (size_t)rx[i].z * A.nzp + zp[i];
+      f[i][0] = *(const v2d *)fa;
+      f[i][2] = *(const v2d *)fb;
+      if (MEAN) {
+        f[i][1] = *(const v2d *)(fa + xs);
+        f[i][3] = *(const v2d *)(fb + xs);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) vn[s] = rho[rr[s]];
+  };
+  auto form = [&](double *d) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      v2d *p = (v2d *)(d + at[i]);
+      p[0] = f[i][0] * f[i][2];
+      if (MEAN) {
+        p[1 * ZT * 32] = f[i][0] * f[i][3];
+        p[2 * ZT * 32] = f[i][1] * f[i][2];
+        p[3 * ZT * 32] = f[i][1] * f[i][3];
+      }
+    }
+  };
+  next(0);
+  load();
+  next(8);
+  form(buf[0]);
+  __syncthreads();
+  int cur = 0;
+  for (int e0 = 0; e0 < n; e0 += 8) {
+    double v[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) v[s] = e0 + 4 * s + mk < n ? vn[s] : 0.0;
+    load();
+    next(e0 + 16);
+    loads_first();
+    const double *d = buf[cur] + lane;
+    if (on)
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        if (s == 0 || e0 + 4 < n)
+#pragma unroll
+          for (int k = 0; k < NX; ++k)
+#pragma unroll
+            for (int t = 0; t < ZT; ++t) C[t][k] = mfma64(v[s], d[((s * NX + k) * ZT + t) * 64], C[t][k]);
+    cur ^= 1;
+    if (e0 + 8 < n) form(buf[cur]);
+    __syncthreads();
+  }
+  if (!on) return;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int yo = y0 + 2 * v + (mk >> 1);           // row 4 v + mk of the product
+    if (yo < A.na && A.act[yo] != A.skip) {
+      double *out = A.zy + (size_t)yo * A.zstride + S.zoff + (size_t)(mk & 1) * A.nz;
+#pragma unroll
+      for (int t = 0; t < ZT; ++t) {
+        const int zt = (blockIdx.z * ZT + t) * 16 + mi;
+        if (zt < A.nz)
+#pragma unroll
+          for (int k = 0; k < NX; ++k) out[(size_t)(2 * k) * A.nz + zt] = C[t][k][v];
+      }
+    }
+  }
+}
+
+// One slot per workgroup, in the order of k_sep_z's workgroups of four.
+template <int ZT, int NW>
+__global__ void __launch_bounds__(64 * NW, ZT > 2 ? 3 : 4) k_sep_z_wide(SepArgs A, const SepSlot *__restrict__ slots,
+                                                                        const int4 *__restrict__ elems) {
+  __shared__ __attribute__((aligned(16))) double buf[2][2 * 4 * ZT * 64];
+  const int x = blockIdx.x & 7, i = blockIdx.x >> 3;
+  const SepSlot S = slots[((i >> 2) * 8 + x) * 4 + (i & 3)];
+  if (S.count == 0) return;
+  if ((S.mat & 1) == 0) sep_z_wide<ZT, NW, true>(A, S, elems, buf);
+  else sep_z_wide<ZT, NW, false>(A, S, elems, buf);
+}
+
 // ---- densities: radial contraction ----------------------------------------------
 struct SepDJob {            // 16-row tiles of one axial pair of one (structure, spins)
   int64_t rd;               // offset of the class's table
