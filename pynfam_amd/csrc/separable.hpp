@@ -817,7 +817,8 @@ __device__ inline void sep_proj_job(const SepArgs &A, const SepPJob &J, int w, i
 // Y[p][(ri, z)] = sum_{c, r} R'_c[r][p] F_c(r, z) on v_mfma_f64_16x16x4: up to RT
 // tiles of 16 slots by CT tiles of 16 (ri, z) per wave, four radial points per
 // step.  The fields are read where k_fields put them.  With many points (RT = 4)
-// the products of a step hide its loads, as in k_sep_dens.  With few, a wave's
+// the products of two steps hide the loads of the next two (N_sh = 16, 128 points
+// 2.01 ms, 2.09 with one; 1.10 at the peak matrix rate).  With few, a wave's
 // chain of steps (some 90) is what takes the time: one slot tile per wave, four
 // steps ahead, and where that leaves the device unfilled one column tile, eight
 // ahead (one point, N_sh = 8: 46 -> 21 us; N_sh = 16: 50 -> 39 us).
@@ -832,10 +833,10 @@ __global__ void __launch_bounds__(64, RT > 1 ? 2 : 3) k_sep_proj(SepArgs A, cons
     return;
   }
   switch (J.nst) {
-    case 1: sep_proj_job<CT, 1, 1>(A, J, w, y); break;
-    case 2: sep_proj_job<CT, 2, 1>(A, J, w, y); break;
-    case 3: sep_proj_job<CT, 3, 1>(A, J, w, y); break;
-    case 4: sep_proj_job<CT, 4, 1>(A, J, w, y); break;
+    case 1: sep_proj_job<CT, 1, 2>(A, J, w, y); break;
+    case 2: sep_proj_job<CT, 2, 2>(A, J, w, y); break;
+    case 3: sep_proj_job<CT, 3, 2>(A, J, w, y); break;
+    case 4: sep_proj_job<CT, 4, 2>(A, J, w, y); break;
     default: break;
   }
 }
