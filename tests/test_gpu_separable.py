@@ -106,3 +106,24 @@ def test_no_product_takes_general_kernels(table):
     for k in range(8):
         assert rel(got[k], ref_h[k]) < 1e-12, k
     eng.close()
+
+
+@pytest.mark.parametrize("ngh,ngl,op,K", [(7, 9, "GT", 0), (22, 13, "RS2", 2), (33, 8, "GT", 1), (65, 6, "F", 0)])
+@pytest.mark.parametrize("npts", [8, 9, 16, 33])
+def test_batch_forms_equal_general_kernels(ngh, ngl, op, K, npts):
+    """The forms for a wave, two and four waves per slot, one to three tiles of
+    axial points and two groups of them, over two iterations from zero: each
+    Hamiltonian agrees to 1e-12 of its largest element (the units' bar), the
+    second one's input is the first one's output, hence 1e-11."""
+    from pynfam_amd.engine import GpuEngine
+    from pynfam_amd.rate import circle_contour
+    prob = problem(6, ngh, ngl, op, K)
+    w = np.asarray(circle_contour(0.0, 6.0, 2 * npts)["z"][:npts])
+    eng = GpuEngine(prob)
+    assert eng.get_option("fp64_separable") == 1
+    got = eng.solve(w, max_iter=3, want_x=True)
+    eng.set_option("fp64_grid", 1)
+    ref = eng.solve(w, max_iter=3, want_x=True)
+    eng.close()
+    assert rel(got["strength"], ref["strength"]) < 1e-11
+    assert rel(got["x"], ref["x"]) < 1e-11
