@@ -2929,8 +2929,8 @@ int tp_prepare(pnfam_gpu_ctx *h) {
 
 // FP64 triple products of a stage, both term sets (re and im): one launch per
 // tile count present, or up to TP_SPLIT_N points one launch of k_triprod_split for
-// all of them (beyond that the groups alone fill the device; N_sh = 16, 4 points:
-// at 4 points 129 us, as much as the launches per count).
+// all of them (beyond that the groups alone fill the device: N_sh = 16, 129 us at
+// 4 points, as much as the launches per count; 42 to 56 us at one).
 int launch_triprod(pnfam_gpu_ctx *h, int stage, const double *bbase, long bstride, double *obase, long ostride, int na,
                    const int *act) {
   const Tp64 M{h->tp_cm64.as<double>(), h->tp_rm64.as<double>(), h->tp_mstride};
@@ -3619,14 +3619,16 @@ bool sep_active(const pnfam_gpu_ctx *h) {
   return h->sep_plan && h->fp64_grid == 0 && !h->basic_kernels && !h->sep_nomem;
 }
 
-// Points a pass of the separable stage takes at once, and the splits of its
-// density contraction: with few points the slots are split so that about 2 048
-// waves run.
 // Projection below eight points: one column tile per wave while that gives at most
 // this many waves (16 per CU; beyond, the operands read once per column tile cost
 // more than the shorter chains save: one point 21 us against 29 at N_sh = 8,
 // 18 against 25 at N_sh = 10).
 constexpr long SEP_PFEW = 4096;
+
+// Points a pass of the separable stage takes at once, and the splits of its
+// density contraction: with few points the slots are split so that about 2 048
+// waves run.  The limit only bounds the memory (N_sh = 16: 20 MB per point; passes
+// of 8 to 128 points take the same time per point).
 constexpr size_t SEP_CHUNK_BYTES = size_t(4) << 30;
 int sep_chunk(const pnfam_gpu_ctx *h, int na) {
   const size_t per = (size_t)std::max(h->sep_zstride, h->sep_ystride) * 8;
