@@ -78,7 +78,11 @@ struct DevPtr {
     if (p && bytes >= n) return 0;
     if (p) { (void)hipFree(p); p = nullptr; bytes = 0; }
     if (n == 0) n = 8;
-    if (hipMalloc(&p, n) != hipSuccess) { p = nullptr; return fail(PNFAM_GPU_ENOMEM, "hipMalloc of " + std::to_string(n) + " bytes failed"); }
+    if (hipMalloc(&p, n) != hipSuccess) {
+      (void)hipGetLastError();   // reported here, not by the next check of a launch as well
+      p = nullptr;
+      return fail(PNFAM_GPU_ENOMEM, "hipMalloc of " + std::to_string(n) + " bytes failed");
+    }
     bytes = n;
     return 0;
   }
@@ -3083,8 +3087,10 @@ int ensure_workspace(pnfam_gpu_ctx *h, int npts, int M) {
     if (h->pin_res) { (void)hipHostFree(h->pin_res); h->pin_res = nullptr; }
     h->pin_cap = 0;
     if (hipHostMalloc((void **)&h->pin_act, 6 * n * 4) != hipSuccess ||
-        hipHostMalloc((void **)&h->pin_res, 4 * n * 8) != hipSuccess)
+        hipHostMalloc((void **)&h->pin_res, 4 * n * 8) != hipSuccess) {
+      (void)hipGetLastError();
       return fail(PNFAM_GPU_ENOMEM, "hipHostMalloc of the pinned staging buffers failed");
+    }
     h->pin_cap = (int)n;
   }
   if ((e = h->d_act.alloc(n * 4))) return e;
