@@ -232,7 +232,14 @@ int pnfam_gpu_calc_hamiltonian_noalloc(pnfam_gpu_ctx *h, const double *d_in, dou
  *                  calc_hamiltonian_noalloc; 1: always the general kernels,
  *                  which contract over all grid points (results differ in
  *                  summation order; read back fp64_separable: 1 where the
- *                  first form is in use);
+ *                  first form is in use, 0 also after a call that took the
+ *                  other one for want of memory);
+ *   fp64_grid_bytes  bytes of the first form's intermediates: a batch that
+ *                  needs more runs in passes of as many points as fit, and
+ *                  where not one fits, or the memory cannot be had, the
+ *                  general kernels run; 0 (default): 4 GiB, at least one point
+ *                  a pass (read back fp64_point_bytes, the bytes of a point,
+ *                  and fp64_held_bytes, what the context holds for the stage);
  *   mix_tau        one-product threshold of the mixed path (PNFAM_GPU_MIX_TAU);
  *   mix_hist64     1: the mixed path keeps its Broyden history in FP64;
  *   mix_drop       0: keep the Broyden pair formed across a refinement;

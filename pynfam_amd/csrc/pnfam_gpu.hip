@@ -73,10 +73,14 @@ __device__ inline v4d mfma64(double a, double b, v4d c) {
 struct DevPtr {
   void *p = nullptr;
   size_t bytes = 0;
-  ~DevPtr() { if (p) (void)hipFree(p); }
+  ~DevPtr() { release(); }
+  void release() {
+    if (p) (void)hipFree(p);
+    p = nullptr; bytes = 0;
+  }
   int alloc(size_t n) {
     if (p && bytes >= n) return 0;
-    if (p) { (void)hipFree(p); p = nullptr; bytes = 0; }
+    release();
     if (n == 0) n = 8;
     if (hipMalloc(&p, n) != hipSuccess) {
       (void)hipGetLastError();   // reported here, not by the next check of a launch as well
@@ -2696,7 +2700,9 @@ struct pnfam_gpu_ctx {
   // FP64 grid stage on product grids (separable.hpp): the basis part, found when
   // the context is created, and the plan of the operator's block structures
   struct SepGroup { int cls, first, count; };   // radial function, members of the state list
-  bool sep_basis = false, sep_plan = false, sep_nomem = false;
+  bool sep_basis = false, sep_plan = false;
+  bool sep_nomem = false;      // the workspace could not be had: the rest of this call takes the general kernels
+  size_t sep_limit = 0;        // option fp64_grid_bytes
   int sep_nz = 0, sep_nr = 0, sep_ncls = 0;
   std::vector<SepGroup> sep_groups;              // per (block, spin), in order of sep_gfirst
   std::vector<int> sep_gfirst;                   // [2 nb + 1]
@@ -3050,8 +3056,7 @@ int launch_triprod_bf16(pnfam_gpu_ctx *h, int stage, const double *bbase, long b
   return 0;
 }
 
-int ensure_workspace(pnfam_gpu_ctx *h, int npts, int M) {
-  if (npts <= h->cap && M == h->hist_cap) return 0;
+int grow_workspace(pnfam_gpu_ctx *h, int npts, int M) {
   // an allocation that fails below leaves its buffer freed: the recorded
   // capacity is cleared first and set only once every buffer is in place
   h->cap = 0;
@@ -3103,6 +3108,22 @@ int ensure_workspace(pnfam_gpu_ctx *h, int npts, int M) {
   h->cap = (int)n;
   h->hist_cap = M;
   return 0;
+}
+
+void sep_release(pnfam_gpu_ctx *h) {
+  h->d_sep_zy.release();
+  h->d_sep_part.release();
+}
+
+int ensure_workspace(pnfam_gpu_ctx *h, int npts, int M) {
+  if (npts <= h->cap && M == h->hist_cap) return 0;
+  int e = grow_workspace(h, npts, M);
+  // the factored grid stage can do without its workspace, a batch cannot
+  if (e == PNFAM_GPU_ENOMEM && h->d_sep_zy.p) {
+    sep_release(h);
+    e = grow_workspace(h, npts, M);
+  }
+  return e;
 }
 
 dim3 grid1(size_t n, int bs, int maxb = 2048) {
@@ -3634,11 +3655,16 @@ constexpr long SEP_PFEW = 4096;
 // Points a pass of the separable stage takes at once, and the splits of its
 // density contraction: with few points the slots are split so that about 2 048
 // waves run.  The limit only bounds the memory (N_sh = 16: 20 MB per point; 128
-// points in passes of 32 take 4 % longer than in one, 64 1 %).
+// points in passes of 32 take 4 % longer than in one, 64 1 %); a pass of one point
+// may exceed it, unless the caller has set the limit (option fp64_grid_bytes): then
+// 0 points a pass, where not even one fits.
 constexpr size_t SEP_CHUNK_BYTES = size_t(4) << 30;
+size_t sep_point_bytes(const pnfam_gpu_ctx *h) {
+  return (size_t)std::max<long>(1, std::max(h->sep_zstride, h->sep_ystride)) * 8;
+}
 int sep_chunk(const pnfam_gpu_ctx *h, int na) {
-  const size_t per = (size_t)std::max(h->sep_zstride, h->sep_ystride) * 8;
-  return (int)std::max<size_t>(1, std::min<size_t>((size_t)na, SEP_CHUNK_BYTES / std::max<size_t>(1, per)));
+  const size_t n = (h->sep_limit ? h->sep_limit : SEP_CHUNK_BYTES) / sep_point_bytes(h);
+  return (int)std::min<size_t>((size_t)na, h->sep_limit ? n : std::max<size_t>(1, n));
 }
 int sep_split(const pnfam_gpu_ctx *h, int nc, bool split) {
   if (!split) return 1;
@@ -3647,14 +3673,17 @@ int sep_split(const pnfam_gpu_ctx *h, int nc, bool split) {
 }
 
 // Device memory of a pass over na points, before any launch (a captured pass
-// cannot allocate).
+// cannot allocate); without it nothing is held.
 int sep_workspace(pnfam_gpu_ctx *h, int na) {
   const int nc = sep_chunk(h, na);
-  if (int e = h->d_sep_zy.alloc((size_t)nc * std::max(h->sep_zstride, h->sep_ystride) * 8)) return e;
   // split counts fall as the points rise: the most partial sums any count up to nc needs
   long parts = 0;
   for (int n = 1; n <= nc; ++n) parts = std::max(parts, (long)n * sep_split(h, n, true));
-  return h->d_sep_part.alloc((size_t)parts * h->sep_arows * 2 * h->sep_nz * 8);
+  int e = nc ? h->d_sep_zy.alloc((size_t)nc * sep_point_bytes(h))
+             : fail(PNFAM_GPU_ENOMEM, "fp64_grid_bytes is below the need of one point");
+  if (!e) e = h->d_sep_part.alloc((size_t)parts * h->sep_arows * 2 * h->sep_nz * 8);
+  if (e) sep_release(h);
+  return e;
 }
 
 // Densities, fields and projection through the separable kernels.
@@ -3752,8 +3781,12 @@ int stage_hamiltonian_sep(pnfam_gpu_ctx *h, int na, const int *act, const GridBu
 int stage_hamiltonian(pnfam_gpu_ctx *h, int na, const int *act) {
   const GridBufs gb{h->d_rsp.as<double>(), 3, 2, h->d_dens.as<double>(), h->d_flds.as<double>(), h->d_hsp.as<double>(),
                     h->few_split_on != 0};
-  // without memory for the separable stage's intermediates the general kernels run
-  if (sep_active(h) && sep_workspace(h, na) == 0) return stage_hamiltonian_sep(h, na, act, gb);
+  // without memory for the separable stage's intermediates the general kernels run,
+  // to the end of the call: an allocation that failed is not tried every iteration
+  if (sep_active(h)) {
+    if (sep_workspace(h, na) == 0) return stage_hamiltonian_sep(h, na, act, gb);
+    h->sep_nomem = true;
+  }
   return stage_hamiltonian_on(h, na, act, gb);
 }
 
@@ -4873,6 +4906,7 @@ static int one_point(pnfam_gpu_ctx *h) {
   if (!h || !h->have_op) return fail(PNFAM_GPU_ESTATE, "no operator set");
   const int R = h->unit_reps;
   h->bs.valid = false;
+  h->sep_nomem = false;
   h->hook_M = -2;
   if (int e = ensure_workspace(h, R, h->hist_cap < 0 ? 1 : h->hist_cap)) return e;
   h->unit_act.resize(R);
@@ -5267,7 +5301,7 @@ static int solve_core(pnfam_gpu_ctx *h, int32_t npts, const double *re_w, const 
     for (int w = 0; w < npts; ++w) nslots += b.done[w] ? 0 : 1;
     if (nslots == 0) { iter = it0; return 0; }
     // (without memory for the separable stage every capture takes the general kernels)
-    h->sep_nomem = sep_active(h) && sep_workspace(h, nslots) != 0;
+    if (sep_active(h) && sep_workspace(h, nslots) != 0) h->sep_nomem = true;
     int *dact = h->d_act.as<int>();
     int *ctl = h->d_gctl.as<int>();
     auto body = [&](int ns) -> int {
@@ -5689,6 +5723,12 @@ int pnfam_gpu_set_option(pnfam_gpu_ctx *h, const char *name, double value) {
   } else if (n == "fp64_grid") {
     if (value != 0 && value != 1) return fail(PNFAM_GPU_EINVAL, "fp64_grid: 0 (separable where the basis allows) or 1 (general)");
     h->fp64_grid = (int)value;
+  } else if (n == "fp64_grid_bytes") {
+    if (!(value >= 0) || value > 1e15 || value != std::floor(value))
+      return fail(PNFAM_GPU_EINVAL, "fp64_grid_bytes: 0 (default) or bytes");
+    h->sep_limit = (size_t)value;
+    h->sep_nomem = false;
+    sep_release(h);
   } else if (n == "proj_stages") {
     if (value != 1 && value != 2) return fail(PNFAM_GPU_EINVAL, "proj_stages: 1 or 2");
     h->proj_ns = (int)value;
@@ -5739,6 +5779,9 @@ int pnfam_gpu_get_option(pnfam_gpu_ctx *h, const char *name, double *value) {
   else if (n == "few_split") *value = h->few_split_on;
   else if (n == "fp64_grid") *value = h->fp64_grid;
   else if (n == "fp64_separable") *value = sep_active(h) ? 1 : 0;
+  else if (n == "fp64_grid_bytes") *value = (double)h->sep_limit;
+  else if (n == "fp64_point_bytes") *value = h->sep_plan ? (double)sep_point_bytes(h) : 0;
+  else if (n == "fp64_held_bytes") *value = (double)(h->d_sep_zy.bytes + h->d_sep_part.bytes);
   else if (n == "graph_launches") *value = (double)h->graph_launches;
   else if (n == "graph_captures") *value = (double)h->graph_captures;
   else if (n == "graph_capture_ms") *value = h->graph_capture_ms;

@@ -34,3 +34,52 @@ def test_failed_allocation_is_reported_once():
     assert np.array_equal(got["iterations"], ref["iterations"])
     assert np.array_equal(got["strength"], ref["strength"])
     eng.close()
+
+
+@pytest.mark.parametrize("graph", [0, 1])
+def test_no_memory_for_the_factored_stage(graph):
+    """A limit below one point's intermediates: solves and per-unit calls give
+    the bits of the kernels over all grid points, and nothing is held; without
+    the limit both take the factored stage again."""
+    from pynfam_amd.engine import GpuEngine
+    eng = GpuEngine(problem(K=1))
+    args = np.random.default_rng(2).standard_normal((8, eng.nxy))
+    eng.set_option("graph", graph)
+    w = contour(5)
+    first, unit = eng.solve(w), eng.calc_hamiltonian(args)
+    assert eng.get_option("fp64_separable") == 1 and eng.get_option("fp64_held_bytes") > 0
+    eng.set_option("fp64_grid_bytes", eng.get_option("fp64_point_bytes") - 1)
+    eng.profile(True)
+    got_unit = eng.calc_hamiltonian(args)
+    classes = eng.kernel_classes()
+    eng.profile(False)
+    assert not any(c.startswith("k_sep_") for c in classes), sorted(classes)
+    got = eng.solve(w)
+    assert eng.get_option("fp64_separable") == 0 and eng.get_option("fp64_held_bytes") == 0
+    eng.set_option("fp64_grid", 1)
+    ref, ref_unit = eng.solve(w), eng.calc_hamiltonian(args)
+    assert np.array_equal(got["strength"], ref["strength"]) and np.array_equal(got["iterations"], ref["iterations"])
+    assert np.array_equal(got_unit, ref_unit)
+    eng.set_option("fp64_grid", 0)
+    # a call that lacked the memory does not bind the ones after it
+    assert np.array_equal(eng.solve(w)["strength"], got["strength"])
+    eng.set_option("fp64_grid_bytes", 0)
+    assert np.array_equal(eng.calc_hamiltonian(args), unit)
+    assert np.array_equal(eng.solve(w)["strength"], first["strength"])
+    assert eng.get_option("fp64_separable") == 1
+    eng.close()
+
+
+def test_batch_takes_the_memory_of_the_factored_stage():
+    """A batch that cannot be allocated gets what the stage holds before it is
+    refused."""
+    from pynfam_amd.engine import GpuEngine
+    eng = GpuEngine(problem())
+    w = contour(3)
+    ref = eng.solve(w)
+    assert eng.get_option("fp64_held_bytes") > 0
+    with pytest.raises(RuntimeError, match="hipMalloc of"):
+        eng.solve(np.full(int(512e9 / (4 * eng.nxy * 8)), 1.0 + 1.0j))
+    assert eng.get_option("fp64_held_bytes") == 0
+    assert np.array_equal(eng.solve(w)["strength"], ref["strength"])
+    eng.close()
