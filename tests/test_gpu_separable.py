@@ -127,3 +127,37 @@ def test_batch_forms_equal_general_kernels(ngh, ngl, op, K, npts):
     eng.close()
     assert rel(got["strength"], ref["strength"]) < 1e-11
     assert rel(got["x"], ref["x"]) < 1e-11
+
+
+@pytest.mark.parametrize("npts,pass_points", [(19, 9), (19, 18), (17, 16), (9, 1), (20, 8)])
+@pytest.mark.parametrize("graph", [0, 1])
+def test_several_passes(npts, pass_points, graph):
+    """A batch in passes of fewer points (option fp64_grid_bytes), the last one of
+    another form: the wave, two-wave and four-wave kernels and the projection's
+    slot tiles add in the same order, so that without the splits of few points
+    the solve has the bits of the one in a single pass; with them (the parts of
+    the densities added in another order) amplitudes after two iterations from
+    zero differ as those of the general kernels do (1e-11, as above)."""
+    from pynfam_amd.engine import GpuEngine
+    from pynfam_amd.rate import circle_contour
+    prob = problem(6, 22, 13, "GT", 1)
+    w = np.asarray(circle_contour(0.0, 6.0, 2 * npts)["z"][:npts])
+    eng = GpuEngine(prob)
+    eng.set_option("graph", graph)
+    for split in (0, 1):
+        eng.set_option("few_split", split)
+        eng.set_option("fp64_grid_bytes", 0)
+        ref = eng.solve(w, max_iter=8 if split == 0 else 3, want_x=True)
+        held = eng.get_option("fp64_held_bytes")
+        eng.set_option("fp64_grid_bytes", pass_points * eng.get_option("fp64_point_bytes"))
+        got = eng.solve(w, max_iter=8 if split == 0 else 3, want_x=True)
+        assert eng.get_option("fp64_separable") == 1 and eng.get_option("fp64_held_bytes") < held
+        assert np.array_equal(got["iterations"], ref["iterations"])
+        if split == 0:
+            assert np.array_equal(got["x"], ref["x"]) and np.array_equal(got["strength"], ref["strength"])
+        else:
+            assert rel(got["x"], ref["x"]) < 1e-11 and rel(got["strength"], ref["strength"]) < 1e-11
+    eng.set_option("fp64_grid", 1)
+    gen = eng.solve(w, max_iter=3, want_x=True)
+    eng.close()
+    assert rel(got["x"], gen["x"]) < 1e-11
