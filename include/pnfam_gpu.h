@@ -221,9 +221,12 @@ int pnfam_gpu_calc_hamiltonian_noalloc(pnfam_gpu_ctx *h, const double *d_in, dou
  *   unit_replicas  1..256: the per-unit entry points run their frequency in
  *                  that many batch slots (identical inputs) and return the last,
  *                  so that they take the launch paths of batches that size;
- *                  once it is given (1 too), the FP64 grid stage of the
- *                  per-unit calls runs the general kernels, whose launch-shape
- *                  options (proj_*, fp64_density) it serves to compare;
+ *                  giving it (1 too) also sets unit_general;
+ *   unit_general   1: the FP64 grid stage of the per-unit calls runs the
+ *                  general kernels, whose launch-shape options (proj_*,
+ *                  fp64_density) unit_replicas serves to compare; 0 (default
+ *                  until unit_replicas is given): the form the solves take
+ *                  (fp64_grid);
  *   fp64_grid      0 (default): on a basis whose wavefunction tables are
  *                  products of a radial and an axial function (found from the
  *                  tables when the context is created; the harmonic-oscillator
@@ -232,7 +235,8 @@ int pnfam_gpu_calc_hamiltonian_noalloc(pnfam_gpu_ctx *h, const double *d_in, dou
  *                  calc_hamiltonian_noalloc; 1: always the general kernels,
  *                  which contract over all grid points (results differ in
  *                  summation order; read back fp64_separable: 1 where the
- *                  first form is in use, 0 also after a call that took the
+ *                  first form is in use -- in per-unit calls only while
+ *                  unit_general is 0 -- and 0 also after a call that took the
  *                  other one for want of memory);
  *   fp64_grid_bytes  bytes of the first form's intermediates: a batch that
  *                  needs more runs in passes of as many points as fit, and

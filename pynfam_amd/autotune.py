@@ -25,10 +25,15 @@ order four of the 28 densities add their same-spin and opposite-spin parts
 (0 against 1: 1e-16 relative) and, for 2, in how the columns of a block are
 grouped into tiles (a few units in the last place of the largest element).
 
-The measurement is the FP64 grid stage (pnfam_gpu_calc_hamiltonian, the
-dominant FP64 cost) on random amplitudes, run in `batch` replica slots so that
-it takes the launch path of batches that size, timed with the engine's
-HIP-event profile, best of `repeats`.  The density and projection kernels are
+These are the shapes of the kernels that contract over all grid points; the
+factored stage, which FP64 solves take on a product basis (fp64_separable reads
+1), has none, so there a tuning changes no solve.
+
+The measurement is the FP64 grid stage over all points
+(pnfam_gpu_calc_hamiltonian) on random amplitudes, run in `batch` replica slots
+so that it takes the launch path of batches that size, timed with the engine's
+HIP-event profile, best of `repeats`; the per-unit calls are left as they were
+(unit_replicas, unit_general).  The density and projection kernels are
 independent, so their options are tuned apart: the density option by the
 density time, the projection options (every combination) by the projection
 time, then proj_freqs_rt1 by the projection time with those applied.
@@ -115,23 +120,26 @@ def tune(eng, batch=64, repeats=3, use_cache=True, seed=0):
     rng = np.random.default_rng(seed)
     # amplitudes of the calc_dHsp_interface argument order; any values serve timing
     args = rng.standard_normal((8, eng.nxy))
-    old_reps = eng.get_option("unit_replicas")
-    eng.set_option("unit_replicas", batch)
-    eng.calc_hamiltonian(args)   # workspace and code objects outside the timing
+    old = [(n, eng.get_option(n)) for n in ("unit_replicas", "unit_general")]   # the first sets the second
     timings, settings = {}, {}
-    eng.set_option("proj_freqs_rt1", 0)
-    for names, kernel in ((DENSITY_OPTIONS, "density"), (PROJECTION_OPTIONS, "project"), (RT1_OPTIONS, "project")):
-        part = {}
-        for combo in itertools.product(*(SPACE[n] for n in names)):
-            for n, v in zip(names, combo):
-                eng.set_option(n, v)
-            part[",".join(f"{n}={v}" for n, v in zip(names, combo))] = _stage_ms(eng, args, repeats, kernel)
-        best = min(part, key=part.get)
-        for kv in best.split(","):
-            settings[kv.split("=")[0]] = int(kv.split("=")[1])
-            eng.set_option(kv.split("=")[0], int(kv.split("=")[1]))
-        timings.update({f"{kernel}:{k}": v for k, v in part.items()})
-    eng.set_option("unit_replicas", old_reps)
+    try:
+        eng.set_option("unit_replicas", batch)
+        eng.calc_hamiltonian(args)   # workspace and code objects outside the timing
+        eng.set_option("proj_freqs_rt1", 0)
+        for names, kernel in ((DENSITY_OPTIONS, "density"), (PROJECTION_OPTIONS, "project"), (RT1_OPTIONS, "project")):
+            part = {}
+            for combo in itertools.product(*(SPACE[n] for n in names)):
+                for n, v in zip(names, combo):
+                    eng.set_option(n, v)
+                part[",".join(f"{n}={v}" for n, v in zip(names, combo))] = _stage_ms(eng, args, repeats, kernel)
+            best = min(part, key=part.get)
+            for kv in best.split(","):
+                settings[kv.split("=")[0]] = int(kv.split("=")[1])
+                eng.set_option(kv.split("=")[0], int(kv.split("=")[1]))
+            timings.update({f"{kernel}:{k}": v for k, v in part.items()})
+    finally:
+        for n, v in old:
+            eng.set_option(n, v)
     rec = {"settings": settings, "ms": timings, "batch": batch, "seconds": time.perf_counter() - t0}
     if use_cache:
         cache[key] = rec

@@ -2685,7 +2685,7 @@ struct pnfam_gpu_ctx {
   // per-unit entry points: batch slots their one frequency runs in (option
   // unit_replicas), so that they take the batched launch paths
   int unit_reps = 1;
-  bool unit_general = false;   // unit_replicas given: the grid stage of the FP64 unit calls runs the general kernels
+  bool unit_general = false;   // the grid stage of the FP64 unit calls runs the general kernels (set with unit_replicas)
   std::vector<int> unit_act;
   // mixed-path options (environment defaults, pnfam_gpu_set_option)
   double mix_tau = 3e-3;        // one-product threshold (PNFAM_GPU_MIX_TAU)
@@ -3706,6 +3706,8 @@ int stage_hamiltonian_sep(pnfam_gpu_ctx *h, int na, const int *act, const GridBu
       const int ns = sep_split(h, nc, gb.split);
       note(h, "k_sep_dens", h->sep_ct[0], ns);
       const int zt = (h->sep_nz + 15) / 16, zg = (zt + 2) / 3;
+      if (nc > 8) note(h, "k_sep_z_wide", nc > 16 ? 4 : 2);
+      else note(h, "k_sep_z");
       const SepSlot *sl = h->d_sep_slots[0].as<SepSlot>();
       const int4 *el = h->d_sep_elems[0].as<int4>();
 #define SEP_Z(ZT)                                                                                                      \
@@ -3764,6 +3766,8 @@ int stage_hamiltonian_sep(pnfam_gpu_ctx *h, int na, const int *act, const GridBu
         default: SEP_P(5); break;
       }
 #undef SEP_P
+      if (nc > 8) note(h, "k_sep_expand_wide", nc > 16 ? 4 : 2);
+      else note(h, "k_sep_expand");
       const SepSlot *sl = h->d_sep_slots[1].as<SepSlot>();
       const int4 *el = h->d_sep_elems[1].as<int4>();
       if (nc > 16)
@@ -5677,6 +5681,9 @@ int pnfam_gpu_set_option(pnfam_gpu_ctx *h, const char *name, double value) {
     if (value < 1 || value > 256 || value != std::floor(value)) return fail(PNFAM_GPU_EINVAL, "unit_replicas in 1..256");
     h->unit_reps = (int)value;
     h->unit_general = true;
+  } else if (n == "unit_general") {
+    if (value != 0 && value != 1) return fail(PNFAM_GPU_EINVAL, "unit_general: 0 or 1");
+    h->unit_general = value != 0;
   } else if (n == "mix_tau") {
     if (!(value >= 0)) return fail(PNFAM_GPU_EINVAL, "mix_tau must be >= 0");
     h->mix_tau = value;
@@ -5753,6 +5760,7 @@ int pnfam_gpu_get_option(pnfam_gpu_ctx *h, const char *name, double *value) {
   if (!h || !name || !value) return fail(PNFAM_GPU_EINVAL, "null argument");
   const std::string n(name);
   if (n == "unit_replicas") *value = h->unit_reps;
+  else if (n == "unit_general") *value = h->unit_general ? 1 : 0;
   else if (n == "mix_tau") *value = h->mix_tau;
   else if (n == "mix_hist64") *value = h->mix_hist64;
   else if (n == "mix_drop") *value = h->mix_drop;
