@@ -2958,7 +2958,10 @@ int launch_triprod(pnfam_gpu_ctx *h, int stage, const double *bbase, long bstrid
     const int nw = split || (ns + 1) % 4 < 2 ? 4 : 2, nz = split ? ns : (ns + nw - 1) / nw;
     const dim3 grid(n, na, nz), block(64 * nw);
     const Group *g = groups + (split ? 0 : h->tpa_first[stage][c]);
+    // the column class, whichever kernel takes it, and the kernel
     note(h, "k_triprod_mfma", std::min(c, TP_MAXCT));
+    if (split) note(h, "k_triprod_split", std::min(c, TP_MAXCT));
+    else note(h, "k_triprod_mfma", std::min(c, TP_MAXCT), nw);
 #define TP_GO(K) \
   hipLaunchKernelGGL(K, grid, block, 0, h->stream, g, terms, M, bbase, bstride, obase, ostride, act, h->nxy, h->skip_slot)
 #define TP_LAUNCH(NC)                                      \

@@ -43,3 +43,38 @@ def test_transforms_at_tile_edges(nsh, op, K, beta):
         for k in range(4):
             assert rel(got[k], ref_q[k]) < 1e-12, (reps, k)
     eng.close()
+
+
+@pytest.mark.parametrize("nsh,K,beta", [(6, 0, 0.0), (16, 1, 0.3)])
+def test_form_by_points(nsh, K, beta):
+    """Up to four points one launch of the split form, over the widest class of a
+    stage; beyond, a launch per column class, four waves to a workgroup or two
+    where four would leave two or three idle.  No other form runs."""
+    from pynfam_amd.engine import GpuEngine
+    from pynfam_amd.problem import build_problem
+    from pynfam_amd.synthetic import synthetic_basis
+    prob = build_problem(synthetic_basis(Z=20, N=28, n00=nsh, beta=beta, ngh=8, ngl=6), "GT", K, "-")
+    db = np.asarray(prob.basis.db)
+    eng = GpuEngine(prob)
+    maps, xy = eng.structures()
+    rng = np.random.default_rng(6)
+    x, hsp = [rng.standard_normal(prob.nxy) for _ in range(4)], rng.standard_normal((8, prob.nxy))
+    for reps in (1, 4, 5, 9):
+        eng.set_option("unit_replicas", reps)
+        for call, blocks in ((lambda: eng.qp2sp(*x), maps), (lambda: eng.sp2qp(hsp), xy)):
+            strips = {}   # column class -> strips of its tallest block
+            for m in blocks:
+                for i, j in enumerate(m):
+                    if j >= 0:
+                        c = (int(db[j]) + 15) // 16
+                        strips[c] = max(strips.get(c, 0), (int(db[i]) + 15) // 16)
+            if reps <= 4:
+                want = {f"k_triprod_split<{max(strips)}>"}
+            else:
+                want = {f"k_triprod_mfma<{c},{4 if s % 4 in (0, 3) else 2}>" for c, s in strips.items()}
+            eng.profile(True)
+            call()
+            got = {c for c in eng.kernel_classes() if c.startswith("k_triprod_split") or "," in c}
+            eng.profile(False)
+            assert got == want, (reps, sorted(got), sorted(want))
+    eng.close()
