@@ -3305,11 +3305,13 @@ int stage_hamiltonian_on(pnfam_gpu_ctx *h, int na, const int *act, const GridBuf
 // ---- FP64 grid stage on product grids (separable.hpp) ------------------------
 constexpr int sep_pad8(int n) { return (n + 7) & ~7; }
 
-// Points along z of the product grid: the divisor of nghl for which the values
-// of a few states are rank-one matrices; 0 if there is none.
-int sep_axial_points(const pnfam_gpu_basis *b) {
+// Points along z of the product grid: the first divisor of nghl, from nz on, for
+// which the values of a few states are rank-one matrices; 0 if there is none.  The
+// few can be rank one for a wrong one too: where they vanish on the outer half of
+// the axis, so they are with half its points.
+int sep_axial_points(const pnfam_gpu_basis *b, int nz) {
   const int G = b->nghl;
-  for (int nz = 2; nz <= G / 2; ++nz) {
+  for (; nz <= G / 2; ++nz) {
     if (G % nz || nz > SEP_MAX1D || G / nz > SEP_MAX1D) continue;
     bool ok = true;
     for (int k = 0; k < 3 && ok; ++k) {
@@ -3328,12 +3330,9 @@ int sep_axial_points(const pnfam_gpu_basis *b) {
   return 0;
 }
 
-// Factors of the wavefunction tables and the radial functions they share.
-// Leaves sep_basis false where the tables are no products.
-int sep_prepare(pnfam_gpu_ctx *h, const pnfam_gpu_basis *b) {
-  const int nz = sep_axial_points(b);
-  if (!nz) return 0;
-  const int nr = b->nghl / nz, D = b->dqp;
+// Factors of the wavefunction tables, nz axial points; *ok: they are products.
+int sep_fit(pnfam_gpu_ctx *h, int nz, std::vector<double> &fr, bool *ok) {
+  const int nr = h->nghl / nz, D = h->dqp;
   DevPtr dfr, dres;
   int e;
   if ((e = dfr.alloc((size_t)D * 4 * nr * 8)) || (e = dres.alloc((size_t)D * 8)) ||
@@ -3346,12 +3345,28 @@ int sep_prepare(pnfam_gpu_ctx *h, const pnfam_gpu_basis *b) {
   S.resid = dres.as<double>();
   hipLaunchKernelGGL(k_sep_fit, dim3(D), dim3(256), 0, h->stream, S);
   HIP_TRY(hipGetLastError());
-  std::vector<double> fr((size_t)D * 4 * nr), res(D);
+  fr.resize((size_t)D * 4 * nr);
+  std::vector<double> res(D);
   HIP_TRY(hipMemcpyAsync(fr.data(), dfr.p, fr.size() * 8, hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(hipMemcpyAsync(res.data(), dres.p, res.size() * 8, hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(hipStreamSynchronize(h->stream));
+  *ok = true;
   for (double r : res)
-    if (!(r <= SEP_TOL)) return 0;
+    if (!(r <= SEP_TOL)) *ok = false;
+  return 0;
+}
+
+// Factors of the wavefunction tables and the radial functions they share.
+// Leaves sep_basis false where the tables are no products.
+int sep_prepare(pnfam_gpu_ctx *h, const pnfam_gpu_basis *b) {
+  std::vector<double> fr;
+  bool ok = false;
+  int nz = 1, e;
+  while (!ok) {
+    if (!(nz = sep_axial_points(b, nz + 1))) return 0;
+    if ((e = sep_fit(h, nz, fr, &ok))) return e;
+  }
+  const int nr = b->nghl / nz, D = b->dqp;
   // radial functions equal to rounding (all four tables) form one class,
   // represented by the mean of its members
   std::vector<int> cls(D), first;

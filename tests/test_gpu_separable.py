@@ -161,3 +161,21 @@ def test_several_passes(npts, pass_points, graph):
     gen = eng.solve(w, max_iter=3, want_x=True)
     eng.close()
     assert rel(got["x"], gen["x"]) < 1e-11
+
+
+@pytest.mark.parametrize("ngh,K", [(96, 0), (100, 1), (128, 0)])
+def test_dense_axial_grid(ngh, K):
+    """Axial points so many that the wavefunctions vanish on the outer half: a few
+    states are products with half the points too, the tables are not.  The real
+    number is found and the factored results meet the oracle."""
+    from pynfam_amd.engine import GpuEngine
+    prob = problem(5, ngh, 6, "GT", K)
+    args, ref_h, ref_d = oracle_case(prob, 11 + K)
+    eng = GpuEngine(prob)
+    assert eng.get_option("fp64_separable") == 1
+    got = eng.calc_hamiltonian(args)
+    for k in range(8):
+        assert rel(got[k], ref_h[k]) < 1e-12, k
+    for sec in (0, 1):
+        assert rel(eng.densities(args, sec), ref_d[sec]) < 1e-12, sec
+    eng.close()
