@@ -237,7 +237,9 @@ int pnfam_gpu_calc_hamiltonian_noalloc(pnfam_gpu_ctx *h, const double *d_in, dou
  *                  summation order; read back fp64_separable: 1 where the
  *                  first form is in use -- in per-unit calls only while
  *                  unit_general is 0 -- and 0 also after a call that took the
- *                  other one for want of memory);
+ *                  other one for want of memory; fp64_residual: largest
+ *                  deviation of the tables from products, relative to each
+ *                  table's largest value, at most 1e-14 for the first form);
  *   fp64_grid_bytes  bytes of the first form's intermediates: a batch that
  *                  needs more runs in passes of as many points as fit, and
  *                  where not one fits, or the memory cannot be had, the

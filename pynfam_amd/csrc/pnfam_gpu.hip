@@ -2703,6 +2703,7 @@ struct pnfam_gpu_ctx {
   bool sep_basis = false, sep_plan = false;
   bool sep_nomem = false;      // the workspace could not be had: the rest of this call takes the general kernels
   size_t sep_limit = 0;        // option fp64_grid_bytes
+  double sep_resid = 1.0;      // largest residual of the tables' product fit
   int sep_nz = 0, sep_nr = 0, sep_ncls = 0;
   std::vector<SepGroup> sep_groups;              // per (block, spin), in order of sep_gfirst
   std::vector<int> sep_gfirst;                   // [2 nb + 1]
@@ -3350,9 +3351,9 @@ int sep_fit(pnfam_gpu_ctx *h, int nz, std::vector<double> &fr, bool *ok) {
   HIP_TRY(hipMemcpyAsync(fr.data(), dfr.p, fr.size() * 8, hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(hipMemcpyAsync(res.data(), dres.p, res.size() * 8, hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(hipStreamSynchronize(h->stream));
-  *ok = true;
-  for (double r : res)
-    if (!(r <= SEP_TOL)) *ok = false;
+  h->sep_resid = 0.0;
+  for (double r : res) h->sep_resid = r <= 1.0 ? std::max(h->sep_resid, r) : 1.0;
+  *ok = h->sep_resid <= SEP_TOL;
   return 0;
 }
 
@@ -3377,7 +3378,7 @@ int sep_prepare(pnfam_gpu_ctx *h, const pnfam_gpu_basis *b) {
       double m = 0.0;
       for (int r = 0; r < nr; ++r) m = std::max(m, std::fabs(v[r]));
       for (int r = 0; r < nr; ++r)
-        if (!(std::fabs(u[r] - v[r]) <= SEP_TOL * m)) return false;
+        if (!(std::fabs(u[r] - v[r]) <= SEP_SAME * m)) return false;
     }
     return true;
   };
@@ -5805,6 +5806,7 @@ int pnfam_gpu_get_option(pnfam_gpu_ctx *h, const char *name, double *value) {
   else if (n == "few_split") *value = h->few_split_on;
   else if (n == "fp64_grid") *value = h->fp64_grid;
   else if (n == "fp64_separable") *value = sep_active(h) ? 1 : 0;
+  else if (n == "fp64_residual") *value = h->sep_resid;
   else if (n == "fp64_grid_bytes") *value = (double)h->sep_limit;
   else if (n == "fp64_point_bytes") *value = h->sep_plan ? (double)sep_point_bytes(h) : 0;
   else if (n == "fp64_held_bytes") *value = (double)(h->d_sep_zy.bytes + h->d_sep_part.bytes);

@@ -25,9 +25,14 @@
 // contract over all points.
 #pragma once
 
-constexpr double SEP_TOL = 3e-14;   // largest residual of a product fit, relative to the table's largest value:
-                                    // the HO tables leave 1e-15 to 4e-15 (their own rounding), any basis whose
-                                    // states are no products leaves 1e-3 or more
+// Largest residual of a product fit, relative to the table's largest value: what a
+// larger one left out would be a change of the caller's tables.  Their own rounding
+// leaves up to 1.9e-15 (HO tables of 2 to 20 shells, 8 x 6 to 120 x 100 points);
+// states that are no products leave 1e-3 or more.
+constexpr double SEP_TOL = 1e-14;
+// Radial functions this close in all four tables are one: the gauge of f4 is the
+// least certain, members of one function differ by up to 9.4e-15 (64 x 64 points).
+constexpr double SEP_SAME = 3e-14;
 constexpr int SEP_MAX1D = 256;      // points per direction the fit's LDS holds
 
 // ---- product fit of the tables ------------------------------------------------

@@ -179,3 +179,22 @@ def test_dense_axial_grid(ngh, K):
     for sec in (0, 1):
         assert rel(eng.densities(args, sec), ref_d[sec]) < 1e-12, sec
     eng.close()
+
+
+def test_small_deviation_takes_general_kernels():
+    """A table 2e-14 of its largest value off a product, ten times what the tables'
+    own rounding leaves: not replaced by its fit."""
+    from pynfam_amd.engine import GpuEngine
+    prob = problem(6, 14, 13, "GT", 0)
+    eng = GpuEngine(prob)
+    assert eng.get_option("fp64_separable") == 1 and 0.0 < eng.get_option("fp64_residual") < 2e-15
+    eng.close()
+    t = prob.basis.wf.copy(order="F")
+    a = int(np.argmax(np.abs(t).max(axis=0)))
+    t[17, a] += 2e-14 * np.abs(t[:, a]).max()
+    prob = copy.copy(prob)
+    prob.basis = copy.copy(prob.basis)
+    prob.basis.wf = t
+    eng = GpuEngine(prob)
+    assert eng.get_option("fp64_separable") == 0
+    eng.close()
