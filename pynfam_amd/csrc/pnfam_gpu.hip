@@ -3429,7 +3429,7 @@ int sep_prepare(pnfam_gpu_ctx *h, const pnfam_gpu_basis *b) {
 int sep_build(pnfam_gpu_ctx *h) {
   h->sep_plan = false;
   if (!h->sep_basis) return 0;
-  const int nz = h->sep_nz, nr = h->sep_nr, W = 2 * nz, nr4 = (nr + 3) & ~3;
+  const int nz = h->sep_nz, nr = h->sep_nr, W = 2 * nz, W8 = 2 * sep_pad8(nz), nr4 = (nr + 3) & ~3;
   const BlockMap *dm[4] = {&h->rspmap[0], &h->rspmap[1], &h->rspmap[3], &h->rspmap[2]};   // rho0, kap0, rho1, kap1
   const BlockMap *pm[4] = {&h->hspmap[0], &h->hspmap[1], &h->hspmap[3], &h->hspmap[2]};   // h0, D0, h1, D1
   const int out_slot[4] = {0, 1, 3, 2};
@@ -3470,6 +3470,15 @@ int sep_build(pnfam_gpu_ctx *h) {
   auto slot_id = [&](const Tab &t, int ca, int cb) {
     return (int)(std::lower_bound(t.keys.begin(), t.keys.end(), std::make_pair(ca, cb)) - t.keys.begin());
   };
+  // a point's Z and Y; their offsets are 32-bit: a larger basis keeps the other kernels
+  // (decided before the first copy, whose sources end with this function)
+  long zall = 0, yall = 0;
+  for (int q = 0; q < 16; ++q) {
+    const bool pair = (q >> 2) & 1;
+    zall += (long)tabs[dtab[q]].keys.size() * (pair ? 1 : SEP_NT) * W;
+    yall += (long)tabs[ptab[q]].keys.size() * (pair ? 1 : SEP_PT) * W8;
+  }
+  if (zall > (1L << 30) || yall > (1L << 30)) return 0;
   std::vector<int2> keys;
   size_t doubles = 0;
   for (auto &t : tabs) {
@@ -3493,7 +3502,6 @@ int sep_build(pnfam_gpu_ctx *h) {
   }
   HIP_TRY(hipGetLastError());
   // column tiles per wave: at most five (20 accumulator tiles)
-  const int W8 = 2 * sep_pad8(nz);
   for (int k = 0; k < 2; ++k) {
     const int nct = ((k ? W8 : W) + 15) / 16;
     h->sep_ncg[k] = (nct + 4) / 5;
@@ -3586,7 +3594,6 @@ int sep_build(pnfam_gpu_ctx *h) {
     // per element: the axial products of the densities and of the expansion
     h->sep_flops_d += (kind ? 4.0 : 16.0) * nz * (double)dm[mat]->nelem(h->db) / 4;
     h->sep_flops_p += (kind ? 4.0 : 20.0) * nz * (double)pm[mat]->nelem(h->db) / 4;
-    if (zoff > (1L << 30) || yoff > (1L << 30)) return 0;   // offsets are 32-bit: such a basis keeps the other kernels
   }
   // the job groups go to the XCD with the least work so far, the costliest group
   // first; lists of unequal length end in empty jobs
