@@ -209,8 +209,9 @@ __global__ void k_tp_pack(const double *__restrict__ m, const int4 *__restrict__
 // the next chunk's loads in flight during the products of this one.  Read
 // straight into the operand layout, a matrix whose rows are contiguous gives
 // every lane a cache line of its own; the L1 then serves one lane a cycle, and
-// that, not the matrix rate, bound the kernel (counters: 0.7 to 0.9 L1 accesses
-// per cycle and CU, 27 to 29 per load, matrix cores busy 43 % of the time).
+// that, not the matrix rate, bound the kernel (counters: 0.6 to 0.7 L1 accesses
+// per cycle and CU, 25 to 28 per load, matrix cores busy 29 to 37 % of the time;
+// now 0.4 to 0.5, 20 to 26 and 63 to 71 %).
 // op(A), with its rows along the lanes, is read from the packed copies.  Buffer
 // loads keep an address in one register, which lets three waves of up to 96
 // columns (four of up to 64) share a SIMD.
@@ -1417,8 +1418,9 @@ __device__ inline cplx mul_i(cplx a) { return {-a.i, a.r}; }   // i*a
 // pnfam_hamiltonian_blas.f90:774-1093 (and 1200-1208 for pairing) resolved per
 // field mf(z, z', s_a, s_b) with s = +1/-1 (index 0/1 here).
 // GRID1D: for the contraction one grid direction at a time, which reads neither the
-// components that are always zero nor (4, 0) and (2, 1), its (0, 4) and +-(1, 2).
-// Stores bound the kernel: half of them for it (N_sh = 16, 128 points 195 -> 110 us).
+// components that are always zero nor (4, 0) and (2, 1), its (0, 4) and +-(1, 2);
+// nor the same-spin (2, 2), its (1, 1), which is stored with the rest.
+// Stores bound the kernel: 68 for it, 180 without (N_sh = 16, 128 points 195 -> 110 us).
 template <bool GRID1D>
 __global__ void __launch_bounds__(128) k_fields(FieldArgs F) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2171,10 +2173,10 @@ __global__ void __launch_bounds__(1024) k_select(const double *__restrict__ si, 
 // H: element type of the history (double; float on the mixed path, whose
 // pending raw vout stays FP64 in pdf, so the residual difference is formed
 // exactly, and whose dv is the step the last update wrote to dvin).
-// The Broyden kernels of an FP64 history run at the memory's rate (6 TB/s at 128
-// points): up to 8 pairs k, 4 + (k + 6) + (k + 5) vectors of 4 nxy pass per
-// iteration in resid, dots and update (7 + (k + 8) + (k + 5) with the difference
-// written here; N_sh = 16, 128 points, this kernel 617 -> 337 us).
+// The Broyden kernels of an FP64 history run at the memory's rate (4.8 to 5.2 TB/s
+// at 128 points, a large copy 4.9): up to 8 pairs k, 4 + (k + 6) + (k + 5) vectors
+// of 4 nxy pass per iteration in resid, dots and update (7 + (k + 8) + (k + 5) with
+// the difference written here; N_sh = 16, 128 points, this kernel 617 -> 337 us).
 template <class H>
 __global__ void __launch_bounds__(BRO_WG) k_bro_resid(BroArgs B) {
   constexpr bool f64 = sizeof(H) == 8;
@@ -2404,7 +2406,7 @@ __global__ void __launch_bounds__(512) k_bro_solve(BroArgs B) {
   __syncthreads();
   // Gauss-Jordan with partial pivoting (the first largest |a[i][c]|).  What a
   // column takes is latency, so it has one barrier (three, and the shuffles of the
-  // search through LDS: 65 us for 30 pairs, now 40): rows stay where they are
+  // search through LDS: 65 us for 50 pairs, now 40): rows stay where they are
   // (lane l of every wave holds the row at position l and swaps it there), every
   // wave finds the pivot by itself, column c and the pivot row are only read in
   // step c (columns up to c are not needed any more), and the pivot row is scaled

@@ -950,7 +950,7 @@ __global__ void __launch_bounds__(256) k_sep_expand(SepArgs A, const SepSlot *__
 // With a wave per slot for 16 frequencies, the products in registers, one wave
 // filled a SIMD's registers and the functions' loads were repeated for every 16
 // points: N_sh = 16, 128 points 2.25 ms, here 1.71 ms (0.40 ms at the peak matrix
-// rate; 2.1 GB read and as much written, 2.4 times what h holds: a slot's elements
+// rate; 4.6 GB read and 2.3 written, 2.7 times what h holds: a slot's elements
 // lie in lines it shares with other slots).
 constexpr int SEP_EW = 4;
 template <int NW, bool MEAN>
